@@ -43,7 +43,8 @@
 //   MFMA core in one workgroup per CU that walks its tiles without stopping
 //   the pipeline between them; half the waves issue the stage loads and the
 //   other half the output stores, so the stores of one tile drain while the
-//   next is multiplied.
+//   next is multiplied.  On 256x256 tiles every wave loads and multiplies
+//   instead, the two waves of a SIMD in turn (gemm_persist_kernel_pp).
 #include <atomic>
 #include <mutex>
 #include <type_traits>
@@ -1673,6 +1674,379 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_persist_kernel(GemmArgs a) 
   }
 }
 
+// ---- persistent prefill kernel on 256x256 tiles: two wave groups a slot apart ---------
+// grid and tile walk as gemm_persist_kernel (one workgroup per CU, an even
+// number of scale groups, tail pieces, grouped tiles).  What bounds that form
+// on these tiles is that a loading wave's multiplies queue behind its own
+// direct-to-LDS loads (the matrix cores were busy 52% of the cycles on
+// 4096x7168x16384), so here every wave loads and multiplies, in turn: a scale
+// group is four slots of a wave,
+//   M0  read the activation operands and half of the first weight half,
+//       issue the weight loads of the next group
+//   C0  multiply the first weight half (read the rest of it on the way)
+//   M1  read the second weight half, issue the activation loads of the group
+//       after next
+//   C1  multiply the second half
+// each closed by a workgroup barrier, and waves 4-7 run one slot behind waves
+// 0-3.  Waves w and w + 4 share a SIMD, so in every slot one of them has the
+// matrix core while the other reads LDS and waits for its loads to issue.
+// The halves of a stage buffer are refilled as soon as both wave groups have
+// read them, so a load has four to six slots to land, with two stage buffers.
+// Reads come before the loads of a slot: loads first or alternating with the
+// reads cost 25% (a direct-to-LDS load holds up the LDS reads behind it).
+//
+// An activation scale costs a whole 128-byte line from L2 (row stride K/32
+// bytes), a third of the kernel's L2 reads when fetched group by group, and
+// the chip runs this kernel at its power limit: the scales of four groups
+// come in one 16-byte load per row (a ring of two such quads).
+//
+// 256x256 tiles, before (gemm_persist_kernel) and now, same box, operands
+// rotated over 1 GiB: 4096x7168x16384 439 -> 419 us, 4096x24576x1536 163 ->
+// 154, 4096^3 63.7 -> 61.1, 32 experts N=4096 K=7168: 8192 rows 386 -> 320,
+// 4096 rows 242 -> 198, 2048 rows 193 -> 174, 1024 rows 179 -> 169; 16
+// experts, 2923 rows, N=7168, K=2048 83 -> 71.
+
+// asm_buffer_to_lds16 unless pred (uniform) is zero; the branch stays inside
+// the assembly, so the code around it remains one block.
+__device__ __forceinline__ void asm_buffer_to_lds16_if(int pred, const u32x4& rsrc, uint32_t lds,
+                                                       int voffset, int soffset) {
+  asm volatile(
+      "s_cmp_eq_u32 %3, 0\n\ts_cbranch_scc1 .Lskip%=\n\ts_nop 4\n\t"
+      "buffer_load_dwordx4 %0, %1, %2 offen lds\n.Lskip%=:"
+      :
+      : "v"(voffset), "s"(rsrc), "s"(soffset), "s"(pred), "{m0}"(lds)
+      : "memory", "scc");
+}
+
+template <int OUT_DT, bool GROUPED = false>
+__global__ __launch_bounds__(512) void gemm_persist_kernel_pp(GemmArgs a) {
+  using OT = typename OutT<OUT_DT>::T;
+  constexpr int BN = 256, BM = 256, TN = 128, TM = 64;
+  constexpr int SN = TN / 16, SM = TM / 16, SH = SN / 2;  // SH: weight slices per half
+  constexpr int kOffA = BN * 128;
+  constexpr int kStage = (BN + BM) * 128 + 1024;
+  constexpr int kQuad = BM * 16 + 1024;  // four groups' activation | weight scales
+  // vmcnt at a slot boundary: the loads a wave may have in flight behind the
+  // ones the next slot reads, without the scale loads (so the wait is never
+  // too weak): before M1 of group g, A(g+1) and B(g+1); before M0 of g+1,
+  // B(g+1)'s second half and A(g+2)
+  constexpr int kBehind0 = 8, kBehind1 = 6;
+  constexpr int kOB = (int)sizeof(OT);
+  constexpr int kRow = 128 + 16;  // padded C row of an output pass in LDS
+  constexpr int kPS = 8 / kOB;    // weight slices per output pass (128 bytes of a C row)
+  constexpr int kEarly = SH / 2;  // weight slices of the first half read in M0
+  __shared__ __attribute__((aligned(1024))) uint8_t smem0[kStage];
+  __shared__ __attribute__((aligned(1024))) uint8_t smem1[kStage];
+  __shared__ __attribute__((aligned(1024))) uint8_t squad[2][kQuad];
+  __shared__ __attribute__((aligned(16))) uint8_t sout[8][16 * kRow];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wn = wave & 1, wm = wave >> 1;
+  const int M = a.m, N = a.n, K = a.k;
+  const int KG = K >> 7;
+  const int NB = (N + 127) >> 7;
+  const int tiles_n = (N + BN - 1) / BN, tiles_m = (M + BM - 1) / BM;
+  const int tiles = tiles_n * (GROUPED ? grouped_mtiles<BM>(a, lane) : tiles_m);
+  const int P = gridDim.x;
+  const int S = (!GROUPED && a.tail_split > 1) ? a.tail_split : 1;
+  const int full = S > 1 ? tiles / P * P : tiles;
+  const int tail = tiles - full;
+  const int units = full + tail * S;
+  int u = xcd_contiguous((int)blockIdx.x, P);
+  if (u >= units) return;
+  const int NP = KG >> 1;
+  // as in gemm_persist_kernel
+  auto unit_at = [&](int uu, int* n0, int* m0, int* mend, int* e, int* gb, int* ge, int* z,
+                     int* tt) {
+    int t = uu, zz = 0, s = 1;
+    *tt = -1;
+    if (uu >= full) {
+      const int v = uu - full;
+      t = full + v % tail;
+      zz = v / tail;
+      s = S;
+      *tt = v % tail;
+    }
+    if constexpr (GROUPED) {
+      (void)grouped_tile<BM>(a, t / tiles_n, lane, e, m0, mend);
+      *n0 = (t % tiles_n) * BN;
+    } else {
+      int tn, tm;
+      tile_of(t, tiles_n, tiles_m, &tn, &tm);
+      *n0 = tn * BN;
+      *m0 = tm * BM;
+      *mend = M;
+      *e = 0;
+    }
+    *z = zz;
+    *gb = 2 * (int)((int64_t)zz * NP / s);
+    *ge = 2 * (int)((int64_t)(zz + 1) * NP / s);
+  };
+
+  const int lrow = lane >> 3;
+  const int loff = lrow * K + ((lane & 7) ^ lrow) * 16;
+  const int rsub = lane & 15, c0 = lane >> 4;
+
+  // waves 0-3 (kFirst) run one slot ahead of waves 4-7; separate copies of the
+  // loop, as they wait for their loads in different slots
+  auto run = [&](auto role) {
+    constexpr bool kFirst = decltype(role)::value;
+    // End of a slot.  Waves 0-3 are about to read after a multiply slot, waves
+    // 4-7 let them after a memory slot: each waits for its own loads there.
+    // The scheduler moves nothing across.
+    auto slot_end = [&](auto mem, auto behind) {
+      constexpr bool kMem = decltype(mem)::value;
+      constexpr int kBehind = decltype(behind)::value;
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("" ::: "memory");
+      if constexpr (kMem) {
+        __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0_imm(kFirst ? 63 : kBehind));
+      } else if constexpr (kFirst) {
+        __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0_imm(kBehind));
+      }
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    constexpr std::integral_constant<bool, true> mem_end{};
+    constexpr std::integral_constant<bool, false> mul_end{};
+    constexpr std::integral_constant<int, kBehind0> half0{};
+    constexpr std::integral_constant<int, kBehind1> half1{};
+
+    // tile buffers: rows past the last row of A or B read as zeros
+    u32x4 rB, rA, rS;
+    int soff;  // per-lane scale row
+    auto set_loads = [&](int n0, int m0, int mend, int e) {
+      const int nrows = min(BN, N - n0), mrows = min(BM, mend - m0);
+      rB = rsrc_words(a.bq + ((int64_t)e * N + n0) * K, (uint32_t)(nrows * K));
+      rA = rsrc_words(a.aq + (int64_t)m0 * K, (uint32_t)(mrows * K));
+      if constexpr (kFirst) {
+        // waves 0-3: 64 activation scale rows each
+        rS = rsrc_words(a.as + (int64_t)m0 * KG, (uint32_t)(mrows * KG * 4));
+        soff = min(wave * 64 + lane, mrows - 1) * KG * 4;
+      } else {
+        // wave 4: the weight scales of the tile's two blocks
+        const int nb = n0 >> 7;
+        rS = rsrc_words(a.bs + ((int64_t)e * NB + nb) * KG, (uint32_t)(min(2, NB - nb) * KG * 4));
+        soff = min(lane & 1, NB - 1 - nb) * KG * 4;
+      }
+    };
+    auto load_b = [&](uint8_t* sb, int blk, int g) {
+      asm_buffer_to_lds16(rB, lds_addr(sb) + blk * 1024, loff, 8 * blk * K + g * 128);
+    };
+    // the activations of group g: 4 loads
+    auto issue_a = [&](uint8_t* sb, int g) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int blk = wave + 8 * r;
+        asm_buffer_to_lds16(rA, lds_addr(sb) + kOffA + blk * 1024, loff, 8 * blk * K + g * 128);
+      }
+    };
+    // the weights of group g: 4 loads, the two blocks' first halves first
+    auto issue_b = [&](uint8_t* sb, int g) {
+      load_b(sb, wave, g);
+      load_b(sb, 16 + wave, g);
+      load_b(sb, 8 + wave, g);
+      load_b(sb, 24 + wave, g);
+    };
+    // the scales of groups g .. g + 3 (those past the unit's end are not used)
+    auto issue_s = [&](int want, int slot, int g) {
+      asm_buffer_to_lds16_if(__builtin_amdgcn_readfirstlane(kFirst ? want : want & (wave == 4)), rS,
+                             lds_addr(squad[0]) + slot * kQuad + (kFirst ? wave * 1024 : BM * 16),
+                             soff, g * 4);
+    };
+
+    f32x4 acc[SN][SM];
+    i32x8 aop[SM], bop[SH];
+    float sab[SM];
+    f32x4 pv[3];
+    auto promote = [&](int i, int j, const f32x4& p) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[i][j][r] = __builtin_fmaf(p[r], sab[j], acc[i][j][r]);
+    };
+    auto read_b = [&](const uint8_t* st, int h, int lo, int hi) {
+#pragma unroll
+      for (int i = lo; i < hi; ++i) bop[i] = lds_operand(st, wn * TN + 16 * (h * SH + i) + rsub, c0);
+    };
+    // one half's products, each promoted two products later
+    auto mul = [&](int h, const uint8_t* st) {
+      __builtin_amdgcn_s_setprio(1);
+      if (h == 0) read_b(st, 0, kEarly, SH);
+#pragma unroll
+      for (int x = 0; x < SH * SM; ++x) {
+        pv[x % 3] = mfma_group(bop[x / SM], aop[x % SM]);
+        if (x >= 2) promote(h * SH + (x - 2) / SM, (x - 2) % SM, pv[(x - 2) % 3]);
+      }
+      if (h == 0 && kEarly < SH) __builtin_amdgcn_sched_group_barrier(0x100, 2 * (SH - kEarly), 0);
+#pragma unroll
+      for (int x = 0; x < SH * SM; ++x) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        if (x >= 2) __builtin_amdgcn_sched_group_barrier(0x2, 4, 0);
+      }
+      __builtin_amdgcn_s_setprio(0);
+    };
+    // the last two products of a half, promoted after the slot boundary
+    auto finish = [&](int h) {
+      promote(h * SH + SH - 1, SM - 2, pv[(SH * SM - 2) % 3]);
+      promote(h * SH + SH - 1, SM - 1, pv[(SH * SM - 1) % 3]);
+    };
+
+    int n0, m0, mend, ex, gb, ge, z, tt;
+    unit_at(u, &n0, &m0, &mend, &ex, &gb, &ge, &z, &tt);
+    set_loads(n0, m0, mend, ex);
+    int slot = 0;  // scale quad being read
+    issue_s(1, slot, gb);
+    issue_a(smem0, gb);
+    issue_b(smem0, gb);
+    issue_a(smem1, gb + 1);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0_imm(kBehind1));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if constexpr (!kFirst) slot_end(mul_end, half1);
+
+    for (;;) {
+      const int nu = u + P;
+      const bool has_next = nu < units;
+      int nn0 = n0, nm0 = m0, nmend = mend, nex = ex, ngb = gb, nge = ge, nz = z, ntt = tt;
+      if (has_next) unit_at(nu, &nn0, &nm0, &nmend, &nex, &ngb, &nge, &nz, &ntt);
+#pragma unroll
+      for (int i = 0; i < SN; ++i)
+#pragma unroll
+        for (int j = 0; j < SM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      const bool busy = !GROUPED || __builtin_amdgcn_readfirstlane(m0 + wm * TM < mend);
+      auto body = [&](auto busy_c) {
+        constexpr bool kBusy = decltype(busy_c)::value;
+        // one scale group from stage st, number qi of its quad; mem0 and mem1
+        // issue the loads of the two memory slots
+        auto group = [&](const uint8_t* st, int qi, auto mem0, auto mem1) {
+          if constexpr (kBusy) {
+            read_b(st, 0, 0, kEarly);
+#pragma unroll
+            for (int j = 0; j < SM; ++j) aop[j] = lds_operand(st + kOffA, wm * TM + 16 * j + rsub, c0);
+            const float* sq = reinterpret_cast<const float*>(squad[0] + slot * kQuad) + qi;
+            const float sb = sq[BM * 4 + 4 * wn];
+#pragma unroll
+            for (int j = 0; j < SM; ++j) sab[j] = sq[4 * (wm * TM + 16 * j + rsub)] * sb;
+          }
+          mem0();
+          slot_end(mem_end, half0);
+          if constexpr (kBusy) mul(0, st);
+          slot_end(mul_end, half0);
+          if constexpr (kBusy) {
+            finish(0);
+            read_b(st, 1, 0, SH);
+          }
+          mem1();
+          slot_end(mem_end, half1);
+          if constexpr (kBusy) mul(1, st);
+          slot_end(mul_end, half1);
+          if constexpr (kBusy) finish(1);
+        };
+        int qi = 0;  // the pair's place in its quad: 0 or 2
+        for (int g = gb; g + 2 < ge; g += 2) {
+          group(smem0, qi, [&] { issue_b(smem1, g + 1); },
+                [&] {
+                  issue_s(qi >> 1, slot ^ 1, g + 2);
+                  issue_a(smem0, g + 2);
+                });
+          group(smem1, qi + 1, [&] { issue_b(smem0, g + 2); }, [&] { issue_a(smem1, g + 3); });
+          slot ^= qi >> 1;
+          qi ^= 2;
+        }
+        group(smem0, qi, [&] { issue_b(smem1, ge - 1); },
+              [&] {
+                // from here the next unit's groups (the last unit reloads its own)
+                set_loads(nn0, nm0, nmend, nex);
+                issue_s(1, slot ^ 1, ngb);
+                issue_a(smem0, ngb);
+              });
+        group(smem1, qi + 1, [&] { issue_b(smem0, ngb); }, [&] { issue_a(smem1, ngb + 1); });
+        slot ^= 1;
+      };
+      if (busy) {
+        body(std::integral_constant<bool, true>{});
+      } else {
+        body(std::integral_constant<bool, false>{});
+      }
+
+      if (tt >= 0) {
+        // a piece of a cut tile, for gemm_tail_reduce_kernel<256, 256, 2, 4>
+        const int64_t base = ((((int64_t)z * tail + tt) * 8 + wave) * (SN * SM)) * 64 + lane;
+        f32x4* part = reinterpret_cast<f32x4*>(a.ws) + base;
+#pragma unroll
+        for (int i = 0; i < SN; ++i)
+#pragma unroll
+          for (int j = 0; j < SM; ++j) part[(i * SM + j) * 64] = acc[i][j];
+        break;
+      }
+      // the output rows leave through the wave's own staging, 16 rows of 128
+      // bytes a pass
+      if (busy) {
+        OT* C = reinterpret_cast<OT*>(a.c);
+        const bool vec = a.vec_ok && (N % (16 / kOB)) == 0;
+        uint8_t* so = sout[wave];
+#pragma unroll
+        for (int j = 0; j < SM; ++j) {
+#pragma unroll
+          for (int p = 0; p < SN / kPS; ++p) {
+#pragma unroll
+            for (int i = 0; i < kPS; ++i) {
+              uint8_t* dst = so + rsub * kRow + (16 * i + 4 * c0) * kOB;
+              const f32x4& v = acc[p * kPS + i][j];
+              if constexpr (kOB == 4) {
+                *reinterpret_cast<f32x4*>(dst) = v;
+              } else {
+                typedef OT ot4 __attribute__((ext_vector_type(4)));
+                *reinterpret_cast<ot4*>(dst) = ot4{to_out<OUT_DT>(v[0]), to_out<OUT_DT>(v[1]),
+                                                   to_out<OUT_DT>(v[2]), to_out<OUT_DT>(v[3])};
+              }
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+              const int r = 8 * q + lrow;
+              const u32x4 piece = *reinterpret_cast<const u32x4*>(so + r * kRow + (lane & 7) * 16);
+              const int m = m0 + wm * TM + 16 * j + r;
+              const int n = n0 + wn * TN + 16 * kPS * p + (lane & 7) * (16 / kOB);
+              if (m < mend && n < N) {
+                OT* dst = C + (int64_t)m * N + n;
+                if (vec && n + 16 / kOB - 1 < N) {
+                  __builtin_nontemporal_store(piece, reinterpret_cast<u32x4*>(dst));
+                } else {
+                  const OT* e = reinterpret_cast<const OT*>(&piece);
+                  for (int r2 = 0; r2 < 16 / kOB && n + r2 < N; ++r2) dst[r2] = e[r2];
+                }
+              }
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          }
+        }
+      }
+      if (!has_next) break;
+      u = nu;
+      n0 = nn0;
+      m0 = nm0;
+      mend = nmend;
+      ex = nex;
+      gb = ngb;
+      ge = nge;
+      z = nz;
+      tt = ntt;
+    }
+    // the first half of the waves meets the second half's last slot; loads of
+    // the group after the last must not outlive the workgroup's LDS
+    if constexpr (kFirst) slot_end(mul_end, half1);
+    __builtin_amdgcn_s_waitcnt(vmcnt_lgkm0_imm(0));
+  };
+  if (wave < 4) {
+    run(std::integral_constant<bool, true>{});
+  } else {
+    run(std::integral_constant<bool, false>{});
+  }
+}
+
 // ---- tail reduction of the persistent kernel ---------------------------------------
 // One thread per (cut tile, wave, pair, lane) slot of the partial layout the
 // persistent kernel stores: the S pieces' four fp32 values are added in piece
@@ -1821,6 +2195,21 @@ struct CfgEntry {
     gemm_tail_reduce_kernel<BN, BM, WN, WM, kFp16>,                                            \
     gemm_tail_reduce_kernel<BN, BM, WN, WM, kBf16>}}
 
+#define PERSIST_PP_CFG(NAME)                                                                   \
+  {3,                                                                                          \
+   256,                                                                                        \
+   256,                                                                                        \
+   8,                                                                                          \
+   NAME,                                                                                       \
+   {gemm_persist_kernel_pp<kFp32>, gemm_persist_kernel_pp<kFp16>, gemm_persist_kernel_pp<kBf16>}, \
+   {gemm_persist_kernel_pp<kFp32, true>, gemm_persist_kernel_pp<kFp16, true>,                  \
+    gemm_persist_kernel_pp<kBf16, true>},                                                      \
+   {nullptr, nullptr, nullptr},                                                                \
+   {nullptr, nullptr, nullptr},                                                                \
+   {gemm_tail_reduce_kernel<256, 256, 2, 4, kFp32>,                                            \
+    gemm_tail_reduce_kernel<256, 256, 2, 4, kFp16>,                                            \
+    gemm_tail_reduce_kernel<256, 256, 2, 4, kBf16>}}
+
 const CfgEntry kCfgs[] = {
     DECODE_CFG(1, 1, 8, "dec_m16_k1_u8"),
     DECODE_CFG(1, 2, 8, "dec_m16_k2_u8"),
@@ -1841,7 +2230,7 @@ const CfgEntry kCfgs[] = {
     DECODE_LDS_CFG(2, 4, "decl_k2_u4"),
     DECODE_LDS_CFG(4, 4, "decl_k4_u4"),
     DECODE_LDS_CFG(8, 4, "decl_k8_u4"),
-    PERSIST_CFG(256, 256, 2, 4, "per_n256_m256_w8"),
+    PERSIST_PP_CFG("per_n256_m256_w8"),
     PERSIST_CFG(256, 128, 4, 2, "per_n256_m128_w8"),
     PERSIST_CFG(128, 128, 2, 2, "per_n128_m128_w4"),
     DECODE_WIDE_GCFG(4, 4, 2, 2, "dw_m64_k4_w2a2"),
