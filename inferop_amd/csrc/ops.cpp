@@ -614,25 +614,46 @@ int quant_gemm_impl(void* c, void* q, void* scales, const void* x, int32_t dt, c
 // the whole K range, so the weights of every expert with rows leave HBM once
 // at the decode kernel's rate (32 experts, N=4096, K=7168: 2 rows per expert
 // 124 us vs 154 us on the persistent 128x128 tiles, 8 rows 165 vs 173 us; at
-// 16 rows 243 vs 174 us).  Beyond that, with an even K / 128, the persistent
-// kernels, whose load pipeline runs on
-// across a workgroup's tiles, stream the experts' weights best whatever the
-// rows: two 128x128 workgroups per CU below about 96 rows per expert, one
-// 256x256 beyond (measured at 32 experts, N=4096, K=7168: 2 rows per expert
-// 153 us on 128x128 vs 155 us on 16-row tiled; 32 rows 178 vs 217 us; 64 rows
-// 191 us vs 239 us on 256x256; 128 rows 251 us on 256x256 vs 286 us on
-// 128x128 and 385 us tiled; 512 rows 592 vs 843 us tiled).  With an odd
-// K / 128 the tiled kernels: 16-row tiles below 16 rows per expert, 32-row
-// below 24, 64-row three-stage below 64, 128x128 beyond.
+// 16 rows 243 vs 174 us), except over a short K (up to 20 scale groups, even)
+// with a 256x256 tile per CU or more, where a stripe's workgroup spends its time
+// filling and draining its rings and the persistent kernels take over from 2
+// rows per expert (16 experts, N=7168, K=2048: 2 rows 55.5 -> 52.6 us, 8 rows
+// 68.5 -> 53.1; 32 experts, N=4096, K=2304: 67.8 -> 59.2, 80.8 -> 63.1; at 32
+// groups the stripes stay ahead, 32 experts, N=7168, K=4096, 8 rows: 198 vs 235).
+// Beyond that, with an even K / 128, the persistent kernels, whose load
+// pipeline runs on across a workgroup's tiles, stream the experts' weights
+// best: two 128x128 workgroups per CU up to 64 rows per expert, one 256x256
+// beyond (32 experts, N=4096, K=7168: 90 rows 217 -> 177 us, 128 rows 287 -> 197; 8
+// experts, 70 rows 83.6 -> 72.1), from 96 rows where the 256x256 tiles leave
+// three quarters of the CUs idle (32 experts, N=512, 90 rows 61.4 vs 67.1).  Where those tiles cover at most half of the CUs
+// (2 * experts * ceil(N / 256) <= CUs) every workgroup walks the whole K of
+// its one tile alone and the weights arrive at half the chip's rate or less:
+// up to 24 rows per expert the wide decode kernel with 32-row tiles then, from
+// 24 scale groups up (8 experts, N=1000, K=7168, 16 rows 52.9 -> 15.1 us; 8
+// experts, N=4096, K=7168: 12 rows 69.4 -> 51.7, 24 rows 70.6 -> 60.2; 16
+// experts, N=2048, K=7168, 24 rows 71.1 -> 67.5; over 12 groups it loses, 16
+// experts, N=2048, K=1536, 16 rows 19.2 vs 20.3).  With an odd K / 128 the
+// tiled kernels: 16-row tiles below 16 rows per expert, 32-row below 24,
+// 64-row three-stage below 64, 128x128 beyond.
 // m: the rows the tile choice is made for (masked layout: the expected rows
 // per expert times the experts); launch_m: the rows the grid is launched over
 // (masked layout: experts * max_m), which the wide decode kernel's grid limit
 // applies to.
-int32_t select_grouped(int64_t m, int64_t launch_m, int64_t k, int64_t num_experts) {
+int32_t select_grouped(int64_t m, int64_t launch_m, int64_t n, int64_t k, int64_t num_experts,
+                       int cus) {
+  if (cus <= 0) cus = 256;
   const int64_t avg = m / (num_experts > 0 ? num_experts : 1);
   const int64_t ne = num_experts < launch_m ? num_experts : launch_m;
-  if (avg <= 8 && 16 * k <= 0x7FFFFFFF && (launch_m + 15) / 16 + ne <= 65535) return kDwM16K4;
-  if ((k / 128) % 2 == 0) return avg < 96 ? kPerN128M128 : kPerN256M256;
+  const int64_t kg = k / 128;
+  const bool even = kg % 2 == 0;
+  const int64_t t256 = num_experts * ((n + 255) / 256);  // one 256-row tile per expert
+  const bool short_k = even && kg <= 20 && t256 >= cus && avg >= 2;
+  if (avg <= 8 && !short_k && 16 * k <= 0x7FFFFFFF && (launch_m + 15) / 16 + ne <= 65535)
+    return kDwM16K4;
+  if (avg > 8 && avg <= 24 && even && kg >= 24 && 2 * t256 <= cus && 32 * k <= 0x7FFFFFFF &&
+      (launch_m + 31) / 32 + ne <= 65535)
+    return kDwM32K4;
+  if (even) return avg <= 64 || (avg < 96 && 4 * t256 <= cus) ? kPerN128M128 : kPerN256M256;
   if (avg < 16) return kPreN128M16S4;
   if (avg < 24) return kPreN128M32S4;
   if (avg < 64) return kPreN128M64S3;
@@ -686,7 +707,8 @@ int masked_impl(void* c, const void* a_q, const void* a_scales, const void* b_q,
   if (!valid_input_dtype(out_dt)) return INFEROP_ERR_DTYPE;
   if (cfg < 0) {
     const int64_t rows = expected_m > 0 ? (expected_m < max_m ? expected_m : max_m) : max_m;
-    cfg = select_grouped(rows * experts, experts * max_m, k, experts);
+    const DeviceEntry* d = current_device();
+    cfg = select_grouped(rows * experts, experts * max_m, n, k, experts, d ? d->cus : 256);
   }
   if (max_m == 0) return INFEROP_OK;
   if (!gemm_device()) return INFEROP_ERR_DEVICE;
@@ -701,9 +723,10 @@ int grouped_impl(void* c, const void* a_q, const void* a_scales, const void* b_q
   if (!grouped_shape_ok(m, n, k, experts, group_size, block_n)) return INFEROP_ERR_SHAPE;
   if (!valid_input_dtype(out_dt)) return INFEROP_ERR_DTYPE;
   if (m == 0) return INFEROP_OK;
-  if (!gemm_device()) return INFEROP_ERR_DEVICE;
+  const DeviceEntry* d = gemm_device();
+  if (!d) return INFEROP_ERR_DEVICE;
   return grouped_launch(c, a_q, a_scales, b_q, b_scales, offsets, m, n, k, experts, 0, out_dt,
-                        select_grouped(m, m, k, experts), stream);
+                        select_grouped(m, m, n, k, experts, d->cus), stream);
 }
 
 }  // namespace
@@ -986,7 +1009,8 @@ extern "C" int inferop_grouped_gemm_select(int64_t m, int64_t n, int64_t k, int6
                                            int32_t* config) {
   if (m < 0 || n <= 0 || k <= 0 || k % 128 != 0 || num_experts <= 0 || !config)
     return INFEROP_ERR_ARGUMENT;
-  *config = select_grouped(m, m, k, num_experts);
+  const DeviceEntry* d = current_device();
+  *config = select_grouped(m, m, n, k, num_experts, d ? d->cus : 256);
   return INFEROP_OK;
 }
 
@@ -997,7 +1021,9 @@ extern "C" int inferop_grouped_gemm_masked_select(int64_t max_m, int64_t n, int6
       (max_m > 0 && num_experts > 0x7FFFFFFF / max_m))
     return INFEROP_ERR_ARGUMENT;
   const int64_t rows = expected_m > 0 ? (expected_m < max_m ? expected_m : max_m) : max_m;
-  *config = select_grouped(rows * num_experts, num_experts * max_m, k, num_experts);
+  const DeviceEntry* d = current_device();
+  *config = select_grouped(rows * num_experts, num_experts * max_m, n, k, num_experts,
+                           d ? d->cus : 256);
   return INFEROP_OK;
 }
 

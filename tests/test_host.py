@@ -429,3 +429,30 @@ def test_masked_selection_checks_the_launch_grid():
     assert sel(4096, 256, 4) != "dw_m16_k4_w3a3"
     assert sel(4096, 256, 4).startswith("per_")
     assert sel(1024, 64, 8) == "dw_m16_k4_w3a3"  # 4096 + 64 rows of workgroups
+
+
+def test_grouped_selection_short_k_and_few_tiles():
+    # the lines of the grouped choice over N and K (256 CUs): a short even K with a
+    # 256x256 tile per CU, and tiles for at most half of the CUs
+    names = [inferop_amd.gemm_config_name(i) for i in range(inferop_amd.gemm_num_configs())]
+    sel = lambda avg, n, k, e: names[inferop_amd.grouped_gemm_select(avg * e, n, k, e)]
+    assert sel(1, 7168, 2048, 16) == "dw_m16_k4_w3a3"
+    assert sel(2, 7168, 2048, 16) == "per_n128_m128_w4"
+    assert sel(8, 7168, 20 * 128, 16) == "per_n128_m128_w4"
+    assert sel(8, 7168, 22 * 128, 16) == "dw_m16_k4_w3a3"
+    assert sel(8, 7168, 19 * 128, 16) == "dw_m16_k4_w3a3"  # odd: no persistent kernel
+    assert sel(8, 2048, 2048, 16) == "dw_m16_k4_w3a3"      # 128 tiles
+    assert sel(9, 4096, 7168, 8) == "dw_m32_k4_w2a2"       # 128 tiles
+    assert sel(24, 4096, 24 * 128, 8) == "dw_m32_k4_w2a2"
+    assert sel(25, 4096, 7168, 8) == "per_n128_m128_w4"
+    assert sel(9, 4096, 22 * 128, 8) == "per_n128_m128_w4"
+    assert sel(9, 4097, 7168, 8) == "per_n128_m128_w4"     # 136 tiles
+    assert sel(64, 4096, 7168, 8) == "per_n128_m128_w4"
+    assert sel(65, 4096, 7168, 8) == "per_n256_m256_w8"
+    assert sel(95, 512, 7168, 32) == "per_n128_m128_w4"    # 64 tiles
+    assert sel(96, 512, 7168, 32) == "per_n256_m256_w8"
+    # the wide kernel's grid limit, ceil(E * max_m / 32) + E rows of workgroups
+    msel = lambda max_m, e, exp: names[inferop_amd.grouped_gemm_masked_select(max_m, 256, 7168, e,
+                                                                              exp)]
+    assert msel(1024, 128, 16) == "dw_m32_k4_w2a2"
+    assert msel(32768, 128, 16) == "per_n128_m128_w4"
