@@ -50,15 +50,34 @@ def _ptr(t) -> int:
     return t.data_ptr()
 
 
+def _first_current_stream() -> int:
+    """The current torch stream (0 without a device), through torch's public
+    calls, which bring its device runtime up; later calls then read the handle
+    directly (0.2 us where torch.cuda.current_stream() builds a Stream object
+    in 2.9 us, of a call whose launch takes 3 us)."""
+    global _current_stream
+    try:
+        import torch
+        if not torch.cuda.is_available():
+            return 0
+        handle = torch.cuda.current_stream().cuda_stream
+    except Exception:  # torch without a device: null stream
+        return 0
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    device = getattr(torch._C, "_cuda_getDevice", None)
+    bad_fork = getattr(torch._C, "_cuda_isInBadFork", None)
+    if raw and device and bad_fork:
+        # a child forked after this point has no device: null stream, as above
+        _current_stream = lambda: 0 if bad_fork() else raw(device())  # noqa: E731
+    return handle
+
+
+_current_stream = _first_current_stream
+
+
 def _stream(stream) -> int:
     if stream is None:
-        try:
-            import torch
-            if torch.cuda.is_available():
-                return torch.cuda.current_stream().cuda_stream
-        except Exception:  # torch without a device: null stream
-            pass
-        return 0
+        return _current_stream()
     if isinstance(stream, int):
         return stream
     return stream.cuda_stream
@@ -273,10 +292,15 @@ def diag_mfma_loop(iters: int, blocks: int, promote: bool, sink, stream=None) ->
 
 
 # ---- tensor-level conveniences ---------------------------------------------------
+_TORCH_DTYPE_CODE = {}
+
+
 def _torch_dtype_code(t) -> dtype:
-    import torch
-    return {torch.float32: dtype.fp32, torch.float16: dtype.fp16,
-            torch.bfloat16: dtype.bf16}[t]
+    if not _TORCH_DTYPE_CODE:
+        import torch
+        _TORCH_DTYPE_CODE.update({torch.float32: dtype.fp32, torch.float16: dtype.fp16,
+                                  torch.bfloat16: dtype.bf16})
+    return _TORCH_DTYPE_CODE[t]
 
 
 def quantize(x, group_size: int = 128, stream=None):
@@ -286,9 +310,10 @@ def quantize(x, group_size: int = 128, stream=None):
     x = x.contiguous()
     q = torch.empty((rows, cols), dtype=torch.uint8, device=x.device)
     s = torch.empty((rows, cols // group_size), dtype=torch.float32, device=x.device)
-    st = quant_fp8_per_token_group(q, s, x, _torch_dtype_code(x.dtype), rows, cols, group_size,
-                                   stream)
-    if st != Status.OK:
+    st = lib().inferop_quant_fp8_per_token_group(
+        q.data_ptr(), s.data_ptr(), x.data_ptr(), _torch_dtype_code(x.dtype), rows, cols,
+        group_size, _stream(stream))
+    if st:
         raise InferopError(st, "quant_fp8_per_token_group")
     return q, s
 
@@ -326,8 +351,9 @@ def gemm(a_q, a_s, b_q, b_s, out_dtype=None, stream=None):
     m, k = a_q.shape
     n = b_q.shape[0]
     c = torch.empty((m, n), dtype=out_dtype, device=a_q.device)
-    st = w8a8_block_fp8_gemm(c, a_q, a_s, b_q, b_s, m, n, k, 128, 128,
-                             _torch_dtype_code(out_dtype), stream)
-    if st != Status.OK:
+    st = lib().inferop_w8a8_block_fp8_gemm(
+        c.data_ptr(), _ptr(a_q), _ptr(a_s), _ptr(b_q), _ptr(b_s), m, n, k, 128, 128,
+        _torch_dtype_code(out_dtype), _stream(stream))
+    if st:
         raise InferopError(st, "w8a8_block_fp8_gemm")
     return c

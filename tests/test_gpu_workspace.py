@@ -110,3 +110,26 @@ def test_workspace_pool_bounds_memory_over_64_streams():
                        timeout=300)
     print(r.stdout[-1000:])
     assert r.returncode == 0 and "ok" in r.stdout, (r.stdout[-2000:], r.stderr[-2000:])
+
+
+@pytest.mark.gpu
+def test_default_stream_is_torchs_current_one():
+    # the stream a call without one runs on: the current torch stream, also
+    # inside a stream context and in another thread
+    import threading
+
+    from inferop_amd import ops
+
+    device()
+    side = torch.cuda.Stream()
+    assert ops._stream(None) == torch.cuda.current_stream().cuda_stream
+    with torch.cuda.stream(side):
+        assert ops._stream(None) == side.cuda_stream != 0
+        seen = []
+        th = threading.Thread(target=lambda: seen.append(
+            (ops._stream(None), torch.cuda.current_stream().cuda_stream)))
+        th.start()
+        th.join()
+        assert seen[0][0] == seen[0][1]
+    assert ops._stream(None) == torch.cuda.current_stream().cuda_stream
+    assert ops._stream(side) == side.cuda_stream and ops._stream(17) == 17
