@@ -31,6 +31,8 @@
 #include <atomic>
 #include <mutex>
 
+#include <type_traits>
+
 #include "device_common.h"
 #include "hip_launch.h"
 #include "quant_group.h"
@@ -750,6 +752,100 @@ __global__ __launch_bounds__(256) void silu_mul_quant_kernel(uint8_t* __restrict
 // out = dt((residual * inv_rms) * weight) quantized per 128-column group
 // (reference/reference.cpp:23-35 for the arithmetic; the sum of squares is a
 // tree over the stored residual values, the reference's is left to right).
+// Rows of up to NT * 8 * KEEP columns: one workgroup per row, the whole row in
+// registers.  HBM-bound (7 bytes per 16-bit element), and what kept the
+// looping kernel below from the rate of a copy was too few loads in flight:
+// its column blocks sit behind branches, so a wave waits for one before it
+// asks for the next.  Here every load of a row, the weight's too, is issued
+// before the first is used: raw buffer accesses bounded at the row's end read
+// zeros and store nothing past it, so there are no branches, and a dead column
+// block adds +0 to the sum and forms groups of its own that are not stored
+// (cols % 128 == 0).  Everything streams (non-temporal), except that fp32 loads are
+// cached, as a lane's two halves of a 32-byte piece come in two loads.
+// Same box, inputs rotated over 1 GiB, us before and now: bf16 4096x7168 45.6
+// -> 36.9 (5.6 TB/s), 1000x7168 15.4 -> 11.4, 64x7168 8.4 -> 4.4, 4096x2048
+// 14.8 -> 12.4, 2048x16384 54.4 -> 42.3, 2048x18432 63.2 -> 47.8; fp32
+// 4096x7168 80.1 -> 72.0.  Rows kept by a workgroup that walks on to the next
+// row with its loads already in flight were no faster (40.6).
+template <int DT, int NT, int KEEP>
+__global__ __launch_bounds__(NT) void add_rmsnorm_quant_row_kernel(
+    void* __restrict__ residual, uint8_t* __restrict__ q, float* __restrict__ scales,
+    const void* __restrict__ x, const void* __restrict__ weight, int cols, float eps) {
+  constexpr int EB = DT == kFp32 ? 4 : 2;
+  constexpr int W = In<DT>::kWords;
+  constexpr int kLoad = DT == kFp32 ? 0 : 2, kStore = 2;  // buffer cache policy: 2 = nt
+  __shared__ float red[NT / 64];
+  const int t = threadIdx.x;
+  const int64_t row = blockIdx.x;
+  const uint32_t bytes = (uint32_t)cols * EB;
+  auto rsrc = [](const void* p, uint32_t n) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)n, 0x00020000);
+  };
+  const __amdgpu_buffer_rsrc_t rr = rsrc(static_cast<uint8_t*>(residual) + row * bytes, bytes);
+  const __amdgpu_buffer_rsrc_t rx = rsrc(static_cast<const uint8_t*>(x) + row * bytes, bytes);
+  const __amdgpu_buffer_rsrc_t rw = rsrc(weight, bytes);
+  const __amdgpu_buffer_rsrc_t rq = rsrc(q + row * cols, (uint32_t)cols);
+  uint32_t keep[KEEP][W], add[KEEP][W], wt[KEEP][W];
+  auto load = [&](uint32_t (&dst)[KEEP][W], const __amdgpu_buffer_rsrc_t& r, auto policy) {
+#pragma unroll
+    for (int it = 0; it < KEEP; ++it)
+#pragma unroll
+      for (int v = 0; v < W; v += 4) {
+        const u32x4 w = __builtin_bit_cast(
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (t + it * NT) * 8 * EB + v * 4, 0,
+                                                         decltype(policy)::value));
+        dst[it][v] = w.x, dst[it][v + 1] = w.y, dst[it][v + 2] = w.z, dst[it][v + 3] = w.w;
+      }
+  };
+  load(keep, rr, std::integral_constant<int, kLoad>{});
+  load(add, rx, std::integral_constant<int, kLoad>{});
+  load(wt, rw, std::integral_constant<int, 0>{});
+  // residual = dt(residual + x), and the squares of the stored values
+  float ss = 0.0f;
+#pragma unroll
+  for (int it = 0; it < KEEP; ++it) {
+    float rv[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) rv[i] = In<DT>::elem(keep[it], i) + In<DT>::elem(add[it], i);
+    pack_dt8<DT>(rv, keep[it]);
+#pragma unroll
+    for (int v = 0; v < W; v += 4)
+      __builtin_amdgcn_raw_buffer_store_b128(
+          u32x4{keep[it][v], keep[it][v + 1], keep[it][v + 2], keep[it][v + 3]}, rr,
+          (t + it * NT) * 8 * EB + v * 4, 0, kStore);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float sv = In<DT>::elem(keep[it], i);
+      ss += sv * sv;
+    }
+  }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) ss += __shfl_xor(ss, o);
+  if ((t & 63) == 0) red[t >> 6] = ss;
+  __syncthreads();
+  ss = 0.0f;
+#pragma unroll
+  for (int i = 0; i < NT / 64; i += 4) ss += (red[i] + red[i + 1]) + (red[i + 2] + red[i + 3]);
+  const float inv = 1.0f / __builtin_sqrtf(ss / (float)cols + eps);
+  // out = dt((residual * inv) * weight), quantized per 128 columns
+#pragma unroll
+  for (int it = 0; it < KEEP; ++it) {
+    const int c = (t + it * NT) * 8;
+    float y[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      y[i] = In<DT>::elem(keep[it], i) * inv * In<DT>::elem(wt[it], i);
+    uint32_t w[W];
+    pack_dt8<DT>(y, w);
+    uint32_t lo, hi;
+    float s;
+    quant_group_lane<DT>(w, lo, hi, s);
+    __builtin_amdgcn_raw_buffer_store_b64(u32x2{lo, hi}, rq, c, 0, kStore);
+    if ((t & 15) == 0 && c < cols) scales[row * (cols >> 7) + (c >> 7)] = s;
+  }
+}
+
+// Longer rows: the columns in blocks of 2048, the first four kept in registers.
 template <int DT>
 __global__ __launch_bounds__(256) void add_rmsnorm_quant_kernel(
     void* __restrict__ residual, uint8_t* __restrict__ q, float* __restrict__ scales,
@@ -761,9 +857,9 @@ __global__ __launch_bounds__(256) void add_rmsnorm_quant_kernel(
   uint8_t* res = reinterpret_cast<uint8_t*>(residual) + row * cols * EB;
   const uint8_t* xr = reinterpret_cast<const uint8_t*>(x) + row * cols * EB;
   // pass 1 stores residual = dt(residual + x) and sums the squares of the
-  // stored values; the first kKeep column blocks (cols <= 8192) keep those
-  // values in registers for pass 2 (as the stored dt words: half the
-  // registers for 16-bit types), longer rows read the rest back
+  // stored values; the first kKeep column blocks keep those values in
+  // registers for pass 2 (as the stored dt words: half the registers for
+  // 16-bit types), the rest is read back
   constexpr int kKeep = 4;
   uint32_t keep[kKeep][In<DT>::kWords];
   float ss = 0.0f;
@@ -957,6 +1053,30 @@ hipError_t launch_add_rmsnorm_quant(void* residual, uint8_t* q, float* scales, c
                                     const void* weight, int64_t rows, int64_t cols, float eps,
                                     hipStream_t st) {
   if (rows > 0x7FFFFFFF) return hipErrorInvalidConfiguration;
+  auto row_kernel = [&](auto nt, auto keep) {
+    constexpr int NT = decltype(nt)::value, KEEP = decltype(keep)::value;
+    hipLaunchKernelGGL((add_rmsnorm_quant_row_kernel<DT, NT, KEEP>), dim3((unsigned)rows),
+                       dim3(NT), 0, st, residual, q, scales, x, weight, (int)cols, eps);
+    return hipGetLastError();
+  };
+  // The fewest column blocks per thread that leave a row to as many waves as
+  // cover its latency: 256 threads up to 6144 columns (bf16 4096x4096 21.8 us,
+  // 29.6 on 1024 threads; 3001x5120 21.5 on 256, 22.4 on 512), 512 up to 16384
+  // (4096x7168 36.9, 38.3 on 256; 300x12288 9.3, 10.0 on 1024), 1024 beyond.
+  constexpr std::integral_constant<int, 1> k1{};
+  constexpr std::integral_constant<int, 2> k2{};
+  constexpr std::integral_constant<int, 3> k3{};
+  constexpr std::integral_constant<int, 4> k4{};
+  constexpr std::integral_constant<int, 256> t256{};
+  constexpr std::integral_constant<int, 512> t512{};
+  constexpr std::integral_constant<int, 1024> t1024{};
+  if (cols <= 2048) return row_kernel(t256, k1);
+  if (cols <= 4096) return row_kernel(t256, k2);
+  if (cols <= 6144) return row_kernel(t256, k3);
+  if (cols <= 8192) return row_kernel(t512, k2);
+  if (cols <= 12288) return row_kernel(t512, k3);
+  if (cols <= 16384) return row_kernel(t512, k4);
+  if (cols <= 24576) return row_kernel(t1024, k3);
   hipLaunchKernelGGL((add_rmsnorm_quant_kernel<DT>), dim3((unsigned)rows), dim3(256), 0, st,
                      residual, q, scales, x, weight, cols, eps);
   return hipGetLastError();

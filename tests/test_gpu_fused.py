@@ -212,6 +212,33 @@ def test_add_rmsnorm_quant_normal_inputs(kind, shape):
     assert (np.abs(deq - y_ref) <= 0.07 * np.abs(y_ref) + np.repeat(s, 128, axis=1) * 2.0 ** -8).all()
 
 
+@pytest.mark.parametrize("kind", ["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("cols", [128, 2048, 2176, 4096, 4224, 6144, 6272, 8192, 8320, 12288,
+                                  12416, 16384, 16512, 24576, 24704])
+def test_add_rmsnorm_quant_row_widths(kind, cols):
+    # both sides of every width at which the row kernels take over from one
+    # another, and one past the last: integer inputs, so the sums are exact in
+    # any order and every byte must agree; the rows around the call stay as they were
+    device()
+    rows = 3
+    g = np.random.default_rng(cols)
+    res = g.integers(-6, 7, (rows + 2, cols)).astype(np.float32)
+    x = g.integers(-6, 7, (rows, cols)).astype(np.float32)
+    w = (g.integers(1, 9, cols) / 8).astype(np.float32)
+    res[1:4, :128] = 0  # a zero group
+    x[:, :128] = 0
+    rd, rexact = _dev(res, kind)
+    xd, xexact = _dev(x, kind)
+    wd, wexact = _dev(w, kind)
+    q, s = _rms_gpu(rd[1:4], xd, wd, kind, rows, cols, 1e-6)
+    r_new, qr, sr = _rms_oracle(rexact[1:4], xexact, wexact, kind, 1e-6)
+    got = _res_values(rd, kind)
+    assert np.array_equal(got[1:4].view(np.uint32), r_new.view(np.uint32))
+    assert np.array_equal(got[[0, 4]], rexact[[0, 4]])
+    assert np.array_equal(s.view(np.uint32), sr.view(np.uint32))
+    assert np.array_equal(q, qr)
+
+
 def test_fused_rejected_calls():
     device()
     S = ia.Status
