@@ -467,9 +467,12 @@ __device__ __forceinline__ void pack_dt8(const float* v, uint32_t* w) {
     for (int i = 0; i < 8; ++i) w[i] = f2u(v[i]);
   } else if constexpr (DT == kBf16) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      w[i] = uint32_t(__builtin_bit_cast(uint16_t, (__bf16)v[2 * i])) |
-             (uint32_t(__builtin_bit_cast(uint16_t, (__bf16)v[2 * i + 1])) << 16);
+    for (int i = 0; i < 4; ++i) {  // one conversion for the two
+      typedef float f32x2 __attribute__((ext_vector_type(2)));
+      typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+      w[i] = __builtin_bit_cast(
+          uint32_t, __builtin_convertvector((f32x2{v[2 * i], v[2 * i + 1]}), bf16x2));
+    }
   } else {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -565,17 +568,6 @@ __device__ __forceinline__ void silu_lds_fill(float* tab) {
   }
 }
 
-// silu(g) for the bf16 gate whose bits are the upper half of gbits.
-__device__ __forceinline__ float silu_bf16_lds(const float* tab, uint32_t gbits) {
-  const uint32_t b = gbits >> 16;
-  const uint32_t e = (b >> 7) & 0xFFu;
-  const uint32_t rel = e - kSiluLdsLoExp;  // wraps for e < 102
-  const float t = tab[((b >> 15) << 12) | ((rel & 31u) << 7) | (b & 0x7Fu)];
-  const float g = u2f(gbits);
-  const float rule = e < kSiluLdsLoExp ? g * 0.5f : ((b >> 15) ? -0.0f : g);
-  return rel < 32u ? t : rule;
-}
-
 // fp16 gates: the slice of silu_table_f16 for exponent fields [11, 17)
 // (2^-4 <= |g| < 4) of both signs, 2 x 6 x 1024 entries, 48 KB (three
 // workgroups per CU), holds all but about 5% of normally distributed gates;
@@ -602,13 +594,61 @@ __device__ __forceinline__ void silu_f16_lds_fill(float* tab) {
   }
 }
 
-// silu(g) for the fp16 gate g (exactly representable in fp16).
-__device__ __forceinline__ float silu_f16_lds(const float* tab, float g) {
-  const uint32_t b = __builtin_bit_cast(uint16_t, (_Float16)g);
-  const uint32_t rel = ((b >> 10) & 31u) - kSiluF16LoExp;  // wraps below the slice
-  return rel < (uint32_t)kSiluF16Exps
-             ? tab[(b >> 15) * (kSiluF16Exps * 1024) + (rel << 10) + (b & 1023u)]
-             : silu_table_f16[b];
+// SiLU of 8 gates, held as raw words w[4], through the LDS slice of their
+// type, two gates at a time: d holds both gates' distances from the first
+// magnitude of the slice (16 bits each, wrapping below it), and the slice
+// index is d plus the negative half's offset, shifted once to the two byte
+// offsets.  A gate outside the slice reads some entry of it and is
+// replaced afterwards: for bf16 gates only when a lane of the wave holds one
+// (the rules, or the full table); fp16's narrower slice leaves a few percent
+// of the gates to the full table.
+template <int DT>
+__device__ __forceinline__ void silu8_lds(const float* tab, const uint32_t* w, float* y) {
+  constexpr uint32_t kFirst = DT == kBf16 ? kSiluLdsLoExp << 7 : kSiluF16LoExp << 10;
+  constexpr uint32_t kHalf = (DT == kBf16 ? kSiluLdsEntries : kSiluF16LdsEntries) / 2;
+  const uint8_t* base = reinterpret_cast<const uint8_t*>(tab);
+  u16x2 d[4];
+  u16x2 far = {0, 0};
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    d[j] = __builtin_bit_cast(u16x2, w[j] & 0x7FFF7FFFu) - u16x2{(uint16_t)kFirst, (uint16_t)kFirst};
+    far = __builtin_elementwise_max(far, d[j]);
+  }
+  const bool outside = max((uint32_t)far.x, (uint32_t)far.y) >= kHalf;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const u16x2 dc = DT == kBf16 ? d[j]
+                                 : __builtin_elementwise_min(
+                                       d[j], u16x2{(uint16_t)(kHalf - 1), (uint16_t)(kHalf - 1)});
+    uint32_t off;
+    if constexpr (DT == kBf16) {
+      // (d & 4095) | sign << 12
+      off = ((w[j] >> 3) & 0x10001000u) | (__builtin_bit_cast(uint32_t, dc) & 0x0FFF0FFFu);
+    } else {
+      const u16x2 neg = __builtin_bit_cast(u16x2, (w[j] >> 15) & 0x00010001u);
+      off = __builtin_bit_cast(uint32_t, (u16x2)(neg * u16x2{(uint16_t)kHalf, (uint16_t)kHalf} + dc));
+    }
+    off <<= 2;  // entries of 4 bytes; both halves stay below 2^16
+    y[2 * j] = *reinterpret_cast<const float*>(base + (off & 0xFFFFu));
+    y[2 * j + 1] = *reinterpret_cast<const float*>(base + (off >> 16));
+  }
+  if constexpr (DT == kBf16) {
+    if (__ballot(outside) == 0) return;
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const uint32_t bits = (i & 1) ? w[i >> 1] >> 16 : w[i >> 1] & 0xFFFFu;
+    if ((uint32_t)((i & 1) ? d[i >> 1].y : d[i >> 1].x) < kHalf) continue;
+    if constexpr (DT == kBf16) {
+      const float g = u2f(bits << 16);
+      const float rule = ((bits >> 7) & 0xFFu) < kSiluLdsLoExp ? g * 0.5f
+                         : (bits >> 15)                         ? -0.0f
+                                                                : g;
+      y[i] = (bits >> 7) == 0x1FFu ? silu_table_bf16[bits] : rule;
+    } else {
+      y[i] = silu_table_f16[bits];
+    }
+  }
 }
 
 // gate_up: [tokens, 2d] dt (bf16 or fp16) -> q [tokens, d] E4M3, scales
@@ -616,7 +656,12 @@ __device__ __forceinline__ float silu_f16_lds(const float* tab, float g) {
 // 48 KB).  Lane layout as silu_mul_quant_kernel (16
 // lanes per 128-output group, 4 groups per wave and step, U steps issued
 // together); NT-thread workgroups stride over the groups so each copies the
-// tables once, and large workgroups let more waves share one copy.
+// tables once, and large workgroups let more waves share one copy.  The
+// vector ALU, not HBM, bounded it (93% busy at 4096x18432 bf16, 36
+// instructions per output): the slice index is formed for two gates at once
+// (silu8_lds) and a lane's token advances by additions rather than a division
+// per step (an output group g of token t starts at element g * 128 + t * d of
+// gate_up).
 template <int DT, int U, int NT>
 __global__ __launch_bounds__(NT) void silu_mul_quant_lds_kernel(uint8_t* __restrict__ q,
                                                                  float* __restrict__ scales,
@@ -636,56 +681,51 @@ __global__ __launch_bounds__(NT) void silu_mul_quant_lds_kernel(uint8_t* __restr
   const int lane = threadIdx.x & 63;
   const int sub = lane & 15;
   const uint32_t wave = threadIdx.x >> 6;
-  for (uint32_t step = blockIdx.x;; step += gridDim.x) {
-    const uint64_t base = ((uint64_t)step * (NT / 64) + wave) * (4 * U);
-    if (base >= ngroups) break;  // uniform over the wave
-    float gv[U][8], uv[U][8];
-    uint32_t t[U], gc[U];
+  // a lane's U groups of a step: token t[u], group gc[u] of it; the next step
+  // is `stride` groups on, stride_t tokens and stride_g groups
+  const uint32_t stride = gridDim.x * (uint32_t)(NT / 64 * 4 * U);
+  const uint32_t stride_t = stride / gpr, stride_g = stride - stride_t * gpr;
+  uint32_t t[U], gc[U];
+  const uint64_t base0 = ((uint64_t)blockIdx.x * (NT / 64) + wave) * (4 * U);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const uint32_t g = (uint32_t)base0 + 4 * u + (lane >> 4);
+    t[u] = g / gpr;
+    gc[u] = g - t[u] * gpr;
+  }
+  for (uint64_t base = base0; base < ngroups; base += stride) {  // uniform over the wave
+    u32x4 gw[U], uw[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint32_t g = (uint32_t)base + 4 * u + (lane >> 4);
-      t[u] = g / gpr;
-      gc[u] = g - t[u] * gpr;
       if (g < ngroups) {
-        const uint16_t* row = gate_up + (uint64_t)t[u] * 2 * d + gc[u] * 128 + sub * 8;
-        load_dt8<DT, true>(row, gv[u]);
-        load_dt8<DT, true>(row + d, uv[u]);
+        const uint16_t* row = gate_up + ((uint64_t)t[u] * d + (uint64_t)g * 128 + sub * 8);
+        gw[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row));
+        uw[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row + d));
       } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) gv[u][i] = uv[u][i] = 0.0f;
+        gw[u] = uw[u] = u32x4{0u, 0u, 0u, 0u};
       }
+      t[u] += stride_t;
+      gc[u] += stride_g;
+      if (gc[u] >= gpr) gc[u] -= gpr, ++t[u];
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint32_t g = (uint32_t)base + 4 * u + (lane >> 4);
+      const uint32_t gs[4] = {gw[u].x, gw[u].y, gw[u].z, gw[u].w};
+      const uint32_t us[4] = {uw[u].x, uw[u].y, uw[u].z, uw[u].w};
       float y[8];
-      if constexpr (DT == kBf16) {
-        bool special = false;
+      silu8_lds<DT>(tab, gs, y);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          y[i] = silu_bf16_lds(tab, f2u(gv[u][i]));
-          special |= (f2u(gv[u][i]) >> 23) == 0x1FFu;
-        }
-        if (special) {
-#pragma unroll
-          for (int i = 0; i < 8; ++i)
-            if ((f2u(gv[u][i]) >> 23) == 0x1FFu) y[i] = silu_table_bf16[f2u(gv[u][i]) >> 16];
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) y[i] = silu_f16_lds(tab, gv[u][i]);
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) y[i] *= uv[u][i];
+      for (int i = 0; i < 8; ++i) y[i] *= In<DT>::elem(us, i);
       uint32_t w[In<DT>::kWords];
       pack_dt8<DT>(y, w);
       uint32_t lo, hi;
       float s;
       quant_group_lane<DT>(w, lo, hi, s);
       if (g < ngroups) {
-        __builtin_nontemporal_store(
-            u32x2{lo, hi},
-            reinterpret_cast<u32x2*>(q + (uint64_t)t[u] * d + gc[u] * 128 + sub * 8));
+        __builtin_nontemporal_store(u32x2{lo, hi},
+                                    reinterpret_cast<u32x2*>(q + (uint64_t)g * 128 + sub * 8));
         if (sub == 0) scales[g] = s;
       }
     }
