@@ -1030,11 +1030,14 @@ hipError_t silu_device_cus(int* cus) {
   return hipSuccess;
 }
 
-// Workgroups per CU of the LDS-table SiLU kernel: four 512-thread
-// workgroups (32 KB of LDS each) hold 32 waves per CU at 58 VGPRs.  Measured
-// on 4096x18432 bf16 (graph of launches over 1.2 GB of inputs): 4 x 256
-// threads 100 us, 8 x 256 (5 resident) 92 us, 2 x 1024 96 us, 4 x 512 84-87
-// us; four steps in flight per wave (94 VGPRs, 5 waves per SIMD) 100 us.
+// Workgroups per CU of the LDS-table SiLU kernel for bf16 gates: four
+// 512-thread workgroups (32 KB of LDS, 47 VGPRs) are resident and hold a CU's
+// 32 waves.  From 16 steps per CU on, eight are launched: the second four start
+// as the first end, at different times, so loads and stores of the
+// workgroups fall apart (4096x18432 67.3 -> 64.2 us; with 8 steps per CU, 900x18432, the
+// second table copies cost more, 16.9 -> 18.0).  Other shapes on 4096x18432, us:
+// 256 threads 67-69, 1024 threads 65-67, one step in flight per wave 69-76,
+// four 68-70.
 constexpr int kSiluLdsWgPerCu = 4;
 
 // The LDS-table kernels take the group count and d as 32-bit values and form
@@ -1070,8 +1073,8 @@ hipError_t launch_silu_mul_quant(uint8_t* q, float* scales, const void* gate_up,
     if (hipError_t e = silu_device_cus(&cus); e != hipSuccess) return e;
     if (ngroups >= (int64_t)kStep * cus && ngroups <= 0xFFFFFFFFll && d <= 0x7FFFFFFF) {
       const int64_t steps = (ngroups + kStep - 1) / kStep;
-      const int64_t blocks = steps < (int64_t)cus * kSiluLdsWgPerCu ? steps
-                                                                     : (int64_t)cus * kSiluLdsWgPerCu;
+      const int64_t full = (int64_t)cus * kSiluLdsWgPerCu * (steps >= 16 * (int64_t)cus ? 2 : 1);
+      const int64_t blocks = steps < full ? steps : full;
       hipLaunchKernelGGL((silu_mul_quant_lds_kernel<kBf16, UL, NT>), dim3((unsigned)blocks), dim3(NT), 0, st,
                          q, scales, static_cast<const uint16_t*>(gate_up), (uint32_t)d,
                          (uint32_t)(d / 128), (uint32_t)ngroups);
