@@ -20,6 +20,12 @@ namespace inferop_hip {
 namespace {
 
 constexpr int kMaxExperts = 1024;
+// Two waves per token up to one token per SIMD (1024 on the chip): beyond, the
+// second wave's copy of the exponentials costs what the overlap saves (256
+// experts, top-8, us with one wave and with two: 64 tokens 4.51 / 4.04, 1024
+// 5.05 / 4.56, 2048 5.73 / 5.67, 4096 7.26 / 8.03; 1024 experts, top-16, 64
+// tokens 12.2 / 10.1).
+constexpr int kSplitTokens = 1024;
 
 __device__ __forceinline__ uint32_t row16_min_u32(uint32_t v) {
   v = min(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, false));
@@ -52,16 +58,23 @@ __device__ __forceinline__ float funkey(uint32_t k) {
   return u2f((k & 0x80000000u) ? (k & 0x7FFFFFFFu) : ~k);
 }
 
-template <int EPL>
-__global__ __launch_bounds__(64) void topk_softmax_kernel(int32_t* __restrict__ ids,
+// With few tokens (SPLIT, top-k up to 64) a token takes two waves: the serial
+// sum and the selection rounds, 2 us each and independent of one another, run
+// side by side, each on its own copy of the probabilities, and meet where the
+// weights are formed.
+template <int EPL, bool SPLIT>
+__global__ __launch_bounds__(SPLIT ? 128 : 64) void topk_softmax_kernel(int32_t* __restrict__ ids,
                                                            float* __restrict__ weights,
                                                            const float* __restrict__ logits,
                                                            int tokens, int num_experts, int topk,
                                                            int renormalize) {
-  // one wave (one token) per workgroup: at 64 tokens four tokens per
+  // one token per workgroup: at 64 tokens four tokens per
   // workgroup took 6.1 us against 5.5 us, at 4096 tokens the two are level
   __shared__ __attribute__((aligned(16))) float sp[kMaxExperts];
-  const int lane = threadIdx.x;
+  __shared__ float sum;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool adds = !SPLIT || wave == 1, selects = !SPLIT || wave == 0;
   const int t = blockIdx.x;
   const float* row = logits + (int64_t)t * num_experts;
   float x[EPL];
@@ -78,7 +91,7 @@ __global__ __launch_bounds__(64) void topk_softmax_kernel(int32_t* __restrict__ 
   for (int j = 0; j < EPL; ++j) {
     const int e = lane + 64 * j;
     p[j] = (float)::exp((double)(x[j] - mx));
-    sp[e] = e < num_experts ? p[j] : 0.0f;  // slots past the last expert add +0
+    if (adds) sp[e] = e < num_experts ? p[j] : 0.0f;  // slots past the last expert add +0
   }
   // l = p[0] + p[1] + ... in index order (the reference's left-to-right sum),
   // the same chain in every lane from broadcast LDS reads: the slots past the
@@ -89,7 +102,7 @@ __global__ __launch_bounds__(64) void topk_softmax_kernel(int32_t* __restrict__ 
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   float l = 0.0f;
-  {
+  if (adds) {
     constexpr int kB = 8;                // f32x4 reads per batch
     constexpr int kN = EPL * 64 / 4;     // f32x4 slots covering EPL * 64 experts
     constexpr int kBatches = (kN + kB - 1) / kB;
@@ -114,6 +127,7 @@ __global__ __launch_bounds__(64) void topk_softmax_kernel(int32_t* __restrict__ 
 #pragma unroll
       for (int i = 0; i < kB; ++i) cur[i] = nxt[i];
     }
+    if (SPLIT && lane == 0) sum = l;
   }
 
   // top-k in the reference's order (probability descending, lower index
@@ -131,7 +145,7 @@ __global__ __launch_bounds__(64) void topk_softmax_kernel(int32_t* __restrict__ 
   uint32_t my_b = 0;  // lane k < 64: bits of choice k's probability
   int32_t my_id = 0;
   float wsum_big = 0.0f;  // topk > 64: the weights' left-to-right sum
-  for (int k = 0; k < topk; ++k) {
+  for (int k = 0; selects && k < topk; ++k) {
     uint32_t best = key[0];
     int jb = 0;
 #pragma unroll
@@ -159,7 +173,7 @@ __global__ __launch_bounds__(64) void topk_softmax_kernel(int32_t* __restrict__ 
       for (int j = 0; j < EPL; ++j)
         if (j == (be >> 6)) key[j] = 0u;
     }
-    if (topk <= 64) {
+    if (SPLIT || topk <= 64) {
       if (lane == k) my_b = bb - 1u, my_id = be;
     } else {
       const float wk = u2f(bb - 1u) / l;
@@ -167,7 +181,12 @@ __global__ __launch_bounds__(64) void topk_softmax_kernel(int32_t* __restrict__ 
       wsum_big += wk;
     }
   }
-  if (topk <= 64) {
+  if constexpr (SPLIT) {
+    __syncthreads();
+    if (!selects) return;
+    l = sum;
+  }
+  if (SPLIT || topk <= 64) {
     // weights p / l, then their left-to-right sum for renormalize
     const float my_w = u2f(my_b) / l;
     float wsum = 0.0f;
@@ -186,8 +205,13 @@ __global__ __launch_bounds__(64) void topk_softmax_kernel(int32_t* __restrict__ 
 template <int EPL>
 hipError_t launch_topk(int32_t* ids, float* weights, const float* logits, int tokens, int e, int k,
                        int renorm, hipStream_t st) {
-  hipLaunchKernelGGL((topk_softmax_kernel<EPL>), dim3((unsigned)tokens), dim3(64), 0,
-                     st, ids, weights, logits, tokens, e, k, renorm);
+  if (k <= 64 && tokens <= kSplitTokens) {
+    hipLaunchKernelGGL((topk_softmax_kernel<EPL, true>), dim3((unsigned)tokens), dim3(128), 0, st,
+                       ids, weights, logits, tokens, e, k, renorm);
+  } else {
+    hipLaunchKernelGGL((topk_softmax_kernel<EPL, false>), dim3((unsigned)tokens), dim3(64), 0, st,
+                       ids, weights, logits, tokens, e, k, renorm);
+  }
   return hipGetLastError();
 }
 

@@ -101,3 +101,22 @@ def test_topk_rejected_calls():
     assert f(ids, w, lg, 4, 8, 9) == S.ERR_SHAPE
     torch.cuda.synchronize()
     assert (ids == -7).all() and (w == -1.0).all()
+
+
+@pytest.mark.parametrize("experts,k", [(8, 1), (64, 64), (65, 7), (128, 65), (256, 8), (384, 8),
+                                       (1024, 16), (1024, 64)])
+def test_topk_two_waves_equal_one(experts, k):
+    # up to 1024 tokens a token takes two waves, beyond (and past top-64) one: the
+    # same rows in both calls give the same bits, ties and -inf rows included
+    device()
+    g = np.random.default_rng(experts + k)
+    lg = (2.0 * g.standard_normal((1025, experts))).astype(np.float32)
+    lg[3] = 0.25
+    lg[5, experts // 2:] = -np.inf
+    lg[7] = np.round(lg[7])
+    for renorm in (True, False):
+        ids, w = _gpu(lg, k, renorm)
+        for t in (1, 9, 1024):
+            ids_t, w_t = _gpu(lg[:t], k, renorm)
+            assert np.array_equal(ids_t, ids[:t])
+            assert np.array_equal(w_t.view(np.uint32), w[:t].view(np.uint32))
