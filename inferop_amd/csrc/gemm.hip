@@ -535,21 +535,28 @@ __host__ __device__ constexpr int wide_scale_cap() { return 16; }
 // AR = 8 (one activation tile, M <= 8 rows per workgroup): a tile is 8 rows,
 // one load per group instead of two; the MFMA's other 8 columns read stale
 // LDS and their outputs are never stored or summed into stored outputs (each
-// output column of the MFMA depends only on its own activation row).
-template <int MT, int WK, int UW, int UA, bool PRE, int OUT_DT, bool GROUPED = false, int NT = 1,
-          int AR = 16>
-__global__ __launch_bounds__(64 * WK) void gemm_decode_wide_kernel(GemmArgs a) {
+// output column of the MFMA depends only on its own activation row).  Grouped
+// tiles choose it per workgroup, by the rows their expert has in the tile.
+
+// LDS bytes of one wave: its two rings and the preloaded scales.
+template <int MT, int UW, int UA, bool PRE, int NT, int AR>
+constexpr int wide_wave_bytes() {
+  return UW * NT * 2048 + UA * (MT * AR * 128 + (PRE ? 0 : 512)) +
+         (PRE ? 16 * MT * wide_scale_cap() * 4 + 256 : 0);
+}
+
+template <int MT, int WK, int UW, int UA, bool PRE, int OUT_DT, int NT, int AR>
+__device__ __forceinline__ void decode_wide_tile(const GemmArgs& a, uint8_t* smem, int n0, int m0,
+                                                 int mend, const uint8_t* bq, const float* bs) {
   static_assert(NT == 1 || NT == 2 || NT == 4 || NT == 8, "stripes inside one weight block");
-  static_assert(NT == 1 || !GROUPED, "grouped mode streams one stripe");
-  static_assert(AR == 16 || (AR == 8 && MT == 1 && !GROUPED), "8-row tiles: one plain tile");
+  static_assert(AR == 16 || (AR == 8 && MT == 1), "8-row tiles: one tile");
   constexpr int kW = NT * 2048;                       // 16 * NT weight rows x 128 B
   constexpr int kCap = wide_scale_cap();
   constexpr int kOffSa = MT * AR * 128;               // in an activation slot (no PRE)
   constexpr int kOffSb = kOffSa + 256;
   constexpr int kA = MT * AR * 128 + (PRE ? 0 : 512); // MT tiles (+ 64 sa + 64 sb)
   constexpr int kSaF = PRE ? 16 * MT * kCap : 0;      // preloaded sa floats, [row][group]
-  constexpr int kScale = PRE ? kSaF * 4 + 256 : 0;    // + up to 64 sb floats
-  constexpr int kWave = UW * kW + UA * kA + kScale;
+  constexpr int kWave = wide_wave_bytes<MT, UW, UA, PRE, NT, AR>();
   constexpr int kPerIter = 2 * NT + (AR / 8) * MT + (PRE ? 0 : 2);  // loads issued per group
   constexpr int kPairs = NT * MT;                     // 16x16 output blocks
   constexpr int kLP = (kPairs + WK - 1) / WK;         // blocks per wave at the end
@@ -557,29 +564,12 @@ __global__ __launch_bounds__(64 * WK) void gemm_decode_wide_kernel(GemmArgs a) {
   static_assert(UW >= UA && UA >= 2 && kWait <= 63, "ring sizes");
   static_assert(MT >= 1 && MT <= 4 && kCap <= 64, "1 to 4 activation tiles");
   static_assert(kPairs * 1024 <= kWave, "the end-of-kernel sum fits in the slots");
-  __shared__ __attribute__((aligned(1024))) uint8_t smem[WK * kWave];
 
   const int lane = threadIdx.x & 63;
   const int wk = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int M = a.m, N = a.n, K = a.k;
+  const int N = a.n, K = a.k;
   const int KG = K >> 7;
   const int NB = (N + 127) >> 7;
-  const int n0 = blockIdx.x * (16 * NT);
-  // activation rows [m0, mend); the expert's weights and scales when grouped
-  int m0, mend;
-  const uint8_t* bq = a.bq;
-  const float* bs = a.bs;
-  if constexpr (GROUPED) {
-    int e, r0, r1;
-    if (!grouped_tile<16 * MT>(a, (int)blockIdx.y, lane, &e, &r0, &r1)) return;
-    m0 = r0;
-    mend = r1;
-    bq += (int64_t)e * N * K;
-    bs += (int64_t)e * NB * KG;
-  } else {
-    m0 = blockIdx.y * (AR * MT);
-    mend = M;
-  }
   // split z (grid z) covers the scale groups [gz0, gz1); the waves split those
   const int split = gridDim.z, z = blockIdx.z;
   const int gz0 = (int)((int64_t)z * KG / split), gz1 = (int)((int64_t)(z + 1) * KG / split);
@@ -612,7 +602,7 @@ __global__ __launch_bounds__(64 * WK) void gemm_decode_wide_kernel(GemmArgs a) {
     if constexpr (PRE) {
       // entry (r, g) at float r * cnt + g: consecutive lanes read consecutive
       // groups of one activation row
-      const int E = 16 * MT * cnt;
+      const int E = AR * MT * cnt;
       for (int t = 0; t * 64 < E; ++t) {
         const int idx = min(t * 64 + lane, E - 1);
         const int r = idx / cnt, g = idx - r * cnt;
@@ -670,7 +660,7 @@ __global__ __launch_bounds__(64 * WK) void gemm_decode_wide_kernel(GemmArgs a) {
 #pragma unroll
         for (int j = 0; j < MT; ++j) {
           const f32x4 pv = mfma_group(wop, lds_operand(A + j * AR * 128, arow, c0));
-          const float sa = PRE ? sa_l[(16 * j + rsub) * cnt + i]
+          const float sa = PRE ? sa_l[(AR * j + arow) * cnt + i]
                                : reinterpret_cast<const float*>(A + kOffSa)[16 * j + rsub];
           const float sc = sa * sb;
 #pragma unroll
@@ -683,7 +673,7 @@ __global__ __launch_bounds__(64 * WK) void gemm_decode_wide_kernel(GemmArgs a) {
 #pragma unroll
         for (int j = 0; j < MT; ++j) {
           aop[j] = lds_operand(A + j * AR * 128, arow, c0);
-          const float sa = PRE ? sa_l[(16 * j + rsub) * cnt + i]
+          const float sa = PRE ? sa_l[(AR * j + arow) * cnt + i]
                                : reinterpret_cast<const float*>(A + kOffSa)[16 * j + rsub];
           sc[j] = sa * sb;
         }
@@ -745,6 +735,42 @@ __global__ __launch_bounds__(64 * WK) void gemm_decode_wide_kernel(GemmArgs a) {
     const int p = wk * kLP + q;
     if (p < kPairs && lane_row && row_of(q) < mend)
       store_out4<OUT_DT>(a, row_of(q), n0 + 16 * (p / MT) + 4 * c0, part[q]);
+  }
+}
+
+template <int MT, int WK, int UW, int UA, bool PRE, int OUT_DT, bool GROUPED = false, int NT = 1,
+          int AR = 16>
+__global__ __launch_bounds__(64 * WK) void gemm_decode_wide_kernel(GemmArgs a) {
+  static_assert((NT == 1 && AR == 16) || !GROUPED, "grouped mode streams one stripe");
+  const int n0 = blockIdx.x * (16 * NT);
+  if constexpr (GROUPED) {
+    // A tile of at most 8 rows of its expert takes an 8-row activation tile
+    // and, in the same LDS, rings one group deeper: MoE decode steps give an
+    // expert a few rows.  32 experts, 64 rows, N=4096, K=7168: 140.2 -> 133.5 us;
+    // 8 experts of 5 rows 45.1 -> 41.6, with N=7168, K=2048 33.8 -> 32.8.
+    // Workgroups that walk several tiles in a smaller grid lost as much on
+    // those smaller shapes as they gained on the first.
+    constexpr bool kShort = MT == 1 && UW == UA;
+    constexpr int kWave = wide_wave_bytes<MT, UW, UA, PRE, NT, 16>();
+    constexpr int kWave8 = kShort ? wide_wave_bytes<1, UW + 1, UA + 1, PRE, NT, 8>() : 0;
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[WK * (kWave > kWave8 ? kWave : kWave8)];
+    const int KG = a.k >> 7;
+    int e, m0, mend;
+    if (!grouped_tile<16 * MT>(a, (int)blockIdx.y, threadIdx.x & 63, &e, &m0, &mend)) return;
+    const uint8_t* bq = a.bq + (int64_t)e * a.n * a.k;
+    const float* bs = a.bs + (int64_t)e * ((a.n + 127) >> 7) * KG;
+    if constexpr (kShort) {
+      if (mend - m0 <= 8) {
+        decode_wide_tile<1, WK, UW + 1, UA + 1, PRE, OUT_DT, NT, 8>(a, smem, n0, m0, mend, bq, bs);
+        return;
+      }
+    }
+    decode_wide_tile<MT, WK, UW, UA, PRE, OUT_DT, NT, 16>(a, smem, n0, m0, mend, bq, bs);
+  } else {
+    __shared__ __attribute__((
+        aligned(1024))) uint8_t smem[WK * wide_wave_bytes<MT, UW, UA, PRE, NT, AR>()];
+    decode_wide_tile<MT, WK, UW, UA, PRE, OUT_DT, NT, AR>(a, smem, n0, blockIdx.y * (AR * MT), a.m,
+                                                          a.bq, a.bs);
   }
 }
 

@@ -81,6 +81,35 @@ def test_grouped_matches_oracle_per_expert(name):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("k", [384, 2048, 2176, 8192, 8320, 16384, 16512])
+@pytest.mark.parametrize("name", ["dw_m16_k4_w3a3", "dw_m16_k8_w3a3"])
+def test_grouped_short_tiles_equal_plain_gemm(name, k):
+    # tiles with at most 8 rows of an expert take 8-row activation tiles; each
+    # output is the same sum in the same order, so the bits are the plain
+    # GEMM's.  Experts that end just below, at and above 8 rows of a tile; K
+    # from fewer groups than waves up to both sides of the 16 groups per wave
+    # whose scales are preloaded (4 and 8 waves: K = 8192 and 16384)
+    device()
+    sizes = [1, 7, 0, 8, 9, 15, 16, 17, 24, 25]
+    n = 40
+    aq, as_, bq, bs, offsets = _experts(sizes, n, k, seed=29)
+    m = int(offsets[-1])
+    g = [to_dev(v) for v in (aq, as_, bq, bs, offsets)]
+    cfg = _cfg(name)
+    print(f"{name} K={k}", flush=True)
+    c = _grouped(*g, m, n, k, "fp32", cfg)
+    for e in range(len(sizes)):
+        r0, r1 = int(offsets[e]), int(offsets[e + 1])
+        if r1 == r0:
+            continue
+        want = torch.empty((r1 - r0, n), dtype=torch.float32, device="cuda:0")
+        assert inferop_amd.w8a8_block_fp8_gemm_config(
+            want, g[0][r0:r1].contiguous(), g[1][r0:r1].contiguous(), g[2][e], g[3][e], r1 - r0, n,
+            k, DT.fp32, cfg, 1) == 0
+        assert torch.equal(c[r0:r1], want), (name, k, e)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("name", GROUPED)
 def test_grouped_equals_plain_gemm_per_segment(name):
     # the grouped kernel is the tiled kernel on the expert's weights with the
