@@ -613,19 +613,20 @@ int quant_gemm_impl(void* c, void* q, void* scales, const void* x, int32_t dt, c
 // workgroup per (16-row weight stripe, expert tile) streams the stripe over
 // the whole K range, so the weights of every expert with rows leave HBM once
 // at the decode kernel's rate (32 experts, N=4096, K=7168: 2 rows per expert
-// 124 us vs 154 us on the persistent 128x128 tiles, 8 rows 165 vs 173 us; at
+// 153 us vs 171 us on the persistent 128x128 tiles, 8 rows 163 vs 171 us; at
 // 16 rows 243 vs 174 us), except over a short K (up to 20 scale groups, even)
 // with a 256x256 tile per CU or more, where a stripe's workgroup spends its time
 // filling and draining its rings and the persistent kernels take over from 2
-// rows per expert (16 experts, N=7168, K=2048: 2 rows 55.5 -> 52.6 us, 8 rows
-// 68.5 -> 53.1; 32 experts, N=4096, K=2304: 67.8 -> 59.2, 80.8 -> 63.1; at 32
-// groups the stripes stay ahead, 32 experts, N=7168, K=4096, 8 rows: 198 vs 235).
+// rows per expert (16 experts, N=7168, K=2048: 2 rows 60.1 -> 51.2 us, 8 rows
+// 64.6 -> 52.0; 32 experts, N=4096, K=2304: 70.9 -> 60.7, 78.4 -> 61.8; at 32
+// groups the stripes stay ahead, 32 experts, N=7168, K=4096, 8 rows: 188 vs 233).
 // Beyond that, with an even K / 128, the persistent kernels, whose load
 // pipeline runs on across a workgroup's tiles, stream the experts' weights
 // best: two 128x128 workgroups per CU up to 64 rows per expert, one 256x256
 // beyond (32 experts, N=4096, K=7168: 90 rows 217 -> 177 us, 128 rows 287 -> 197; 8
 // experts, 70 rows 83.6 -> 72.1), from 96 rows where the 256x256 tiles leave
-// three quarters of the CUs idle (32 experts, N=512, 90 rows 61.4 vs 67.1).  Where those tiles cover at most half of the CUs
+// three quarters of the CUs idle (32 experts, N=512, 90 rows 61.4 vs 67.1).
+// Where those tiles cover at most half of the CUs
 // (2 * experts * ceil(N / 256) <= CUs) every workgroup walks the whole K of
 // its one tile alone and the weights arrive at half the chip's rate or less:
 // up to 24 rows per expert the wide decode kernel with 32-row tiles then, from
