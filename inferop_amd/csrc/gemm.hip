@@ -749,7 +749,8 @@ __global__ __launch_bounds__(64 * WK) void gemm_decode_wide_kernel(GemmArgs a) {
     // expert a few rows.  32 experts, 64 rows, N=4096, K=7168: 140.2 -> 133.5 us;
     // 8 experts of 5 rows 45.1 -> 41.6, with N=7168, K=2048 33.8 -> 32.8.
     // Workgroups that walk several tiles in a smaller grid lost as much on
-    // those smaller shapes as they gained on the first.
+    // those smaller shapes as they gained on the first (with a grid that held
+    // max_m / 16 + 1 tiles per expert).
     constexpr bool kShort = MT == 1 && UW == UA;
     constexpr int kWave = wide_wave_bytes<MT, UW, UA, PRE, NT, 16>();
     constexpr int kWave8 = kShort ? wide_wave_bytes<1, UW + 1, UA + 1, PRE, NT, 8>() : 0;
@@ -2756,6 +2757,14 @@ extern "C" int inferop_hip_gemm_w8a8_block_grouped(void* c, const uint8_t* a_q,
   const int64_t tn = (n + cf.bn - 1) / cf.bn;
   const int64_t tmv = (m + cf.bm - 1) / cf.bm + (experts < m ? experts : m);
   if (tn * tmv > 0x7FFFFFFF) return hipErrorInvalidConfiguration;
+  // masked layout: an expert's count is clamped to max_m, so it has at most
+  // ceil(max_m / BM) tiles whatever the counts are; a workgroup launched for a
+  // tile that turns out empty costs 1.2 ns (the wide kernel with the grid above
+  // and with this one, 64 rows, 32 experts, N=4096, K=7168: max_m 8 135.5 ->
+  // 130.9 us, 16 141.1 -> 131.3, 32 151.9 -> 141.3, 128 216.4 -> 205.6; 8
+  // experts, 40 rows, max_m 16, N=7168, K=2048 35.9 -> 31.5)
+  const int64_t cap = experts * ((max_m + cf.bm - 1) / cf.bm);
+  const int64_t launch_tmv = max_m > 0 && cap < tmv ? cap : tmv;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int out_bytes = out_dt == kFp32 ? 4 : 2;
   const int vec_ok = (n % 4 == 0) && ((uintptr_t)c % (size_t)(4 * out_bytes) == 0);
@@ -2767,10 +2776,10 @@ extern "C" int inferop_hip_gemm_w8a8_block_grouped(void* c, const uint8_t* a_q,
     if (16 * k > 0x7FFFFFFF || tmv > 65535) return hipErrorInvalidConfiguration;
     const int64_t per_wave = (k / 128 + cf.waves - 1) / cf.waves;
     const KernelFn fn = per_wave <= wide_scale_cap() ? cf.fn_grp[di] : cf.fn_grp_alt[di];
-    hipLaunchKernelGGL(fn, dim3((unsigned)tn, (unsigned)tmv), dim3(64 * cf.waves), 0, st, args);
+    hipLaunchKernelGGL(fn, dim3((unsigned)tn, (unsigned)launch_tmv), dim3(64 * cf.waves), 0, st, args);
     return hipGetLastError();
   }
-  int64_t grid = tn * tmv;
+  int64_t grid = tn * launch_tmv;
   if (cf.kind == 3) {
     // persistent: one workgroup per CU (two for 128x128 tiles) walks the
     // tiles, whose number the kernel takes from the offsets

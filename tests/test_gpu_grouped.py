@@ -243,6 +243,33 @@ def test_grouped_masked_layout(name):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("max_m", [1, 8, 16, 17])
+@pytest.mark.parametrize("name", GROUPED)
+def test_grouped_masked_grid_holds_full_experts(name, max_m):
+    # the grid holds experts * ceil(max_m / tile rows) tiles at most: with every
+    # expert full (one count past max_m) the last expert's last tile is in it
+    device()
+    counts = [max_m] * 5
+    n, k = 72, 512
+    aq, as_, bq, bs, offsets = _experts(counts, n, k, seed=31 + max_m)
+    a3, s3 = _masked_inputs(counts, max_m, aq, as_, offsets)
+    cfg = _cfg(name)
+    B, BS = to_dev(bq), to_dev(bs)
+    flat = _grouped(to_dev(aq), to_dev(as_), B, BS, to_dev(offsets), int(offsets[-1]), n, k,
+                    "fp32", cfg)
+    c3 = torch.full((len(counts), max_m, n), float("nan"), device="cuda:0")
+    given = np.array(counts[:-1] + [max_m + 100], np.int32)
+    assert inferop_amd.w8a8_block_fp8_grouped_gemm_masked_config(
+        c3, to_dev(a3), to_dev(s3), B, BS, to_dev(given), max_m, n, k, len(counts), DT.fp32,
+        cfg) == 0
+    assert torch.equal(c3.reshape(-1, n), flat)
+    for e in (0, 4):
+        r0 = int(offsets[e])
+        assert_gemm_close(out_to_f32(c3[e]), oracle.gemm(aq[r0:r0 + max_m], as_[r0:r0 + max_m],
+                                                         bq[e], bs[e]), f"{name} expert {e}")
+
+
+@pytest.mark.gpu
 def test_grouped_masked_counts_clamped_and_hint():
     # counts are device data: negative counts act as 0 and counts past max_m
     # as max_m; expected_m only steers the tile choice (the result is the same
