@@ -739,7 +739,7 @@ __device__ __forceinline__ void decode_wide_tile(const GemmArgs& a, uint8_t* sme
 }
 
 template <int MT, int WK, int UW, int UA, bool PRE, int OUT_DT, bool GROUPED = false, int NT = 1,
-          int AR = 16>
+          int AR = 16, bool WALK = false>
 __global__ __launch_bounds__(64 * WK) void gemm_decode_wide_kernel(GemmArgs a) {
   static_assert((NT == 1 && AR == 16) || !GROUPED, "grouped mode streams one stripe");
   const int n0 = blockIdx.x * (16 * NT);
@@ -748,25 +748,35 @@ __global__ __launch_bounds__(64 * WK) void gemm_decode_wide_kernel(GemmArgs a) {
     // and, in the same LDS, rings one group deeper: MoE decode steps give an
     // expert a few rows.  32 experts, 64 rows, N=4096, K=7168: 140.2 -> 133.5 us;
     // 8 experts of 5 rows 45.1 -> 41.6, with N=7168, K=2048 33.8 -> 32.8.
-    // Workgroups that walk several tiles in a smaller grid lost as much on
-    // those smaller shapes as they gained on the first (with a grid that held
-    // max_m / 16 + 1 tiles per expert).
     constexpr bool kShort = MT == 1 && UW == UA;
     constexpr int kWave = wide_wave_bytes<MT, UW, UA, PRE, NT, 16>();
     constexpr int kWave8 = kShort ? wide_wave_bytes<1, UW + 1, UA + 1, PRE, NT, 8>() : 0;
     __shared__ __attribute__((aligned(1024))) uint8_t smem[WK * (kWave > kWave8 ? kWave : kWave8)];
     const int KG = a.k >> 7;
-    int e, m0, mend;
-    if (!grouped_tile<16 * MT>(a, (int)blockIdx.y, threadIdx.x & 63, &e, &m0, &mend)) return;
-    const uint8_t* bq = a.bq + (int64_t)e * a.n * a.k;
-    const float* bs = a.bs + (int64_t)e * ((a.n + 127) >> 7) * KG;
-    if constexpr (kShort) {
-      if (mend - m0 <= 8) {
-        decode_wide_tile<1, WK, UW + 1, UA + 1, PRE, OUT_DT, NT, 8>(a, smem, n0, m0, mend, bq, bs);
-        return;
+    // WALK: a workgroup goes on by the grid's height through the masked
+    // experts' tiles
+    const int last = WALK ? a.experts * ((a.max_m + 16 * MT - 1) / (16 * MT)) : 0;
+    for (int t = blockIdx.y;;) {
+      int e, m0, mend;
+      if (!grouped_tile<16 * MT>(a, t, threadIdx.x & 63, &e, &m0, &mend)) return;
+      const uint8_t* bq = a.bq + (int64_t)e * a.n * a.k;
+      const float* bs = a.bs + (int64_t)e * ((a.n + 127) >> 7) * KG;
+      bool done = false;
+      if constexpr (kShort) {
+        if (mend - m0 <= 8) {
+          decode_wide_tile<1, WK, UW + 1, UA + 1, PRE, OUT_DT, NT, 8>(a, smem, n0, m0, mend, bq,
+                                                                      bs);
+          if constexpr (!WALK) return;
+          done = true;
+        }
       }
+      if (!done)
+        decode_wide_tile<MT, WK, UW, UA, PRE, OUT_DT, NT, 16>(a, smem, n0, m0, mend, bq, bs);
+      if constexpr (!WALK) return;
+      t += gridDim.y;
+      if (t >= last) return;
+      __syncthreads();  // the tile's sums have been read from the rings' LDS
     }
-    decode_wide_tile<MT, WK, UW, UA, PRE, OUT_DT, NT, 16>(a, smem, n0, m0, mend, bq, bs);
   } else {
     __shared__ __attribute__((
         aligned(1024))) uint8_t smem[WK * wide_wave_bytes<MT, UW, UA, PRE, NT, AR>()];
@@ -2123,6 +2133,9 @@ struct CfgEntry {
   KernelFn fn_grp_alt[3];
   // persistent (kind 3): the reduction of cut tail tiles
   void (*fn_tail[3])(GemmArgs, int, int);
+  // wide decode (kind 4): fn_grp and fn_grp_alt walking a lower grid
+  KernelFn fn_walk[3];
+  KernelFn fn_walk_alt[3];
 };
 
 #define DECODE_CFG(MT, WK, U, NAME)                                                           \
@@ -2180,7 +2193,14 @@ struct CfgEntry {
     gemm_decode_wide_kernel<MT, WK, UW, UA, true, kBf16, true>},                               \
    {gemm_decode_wide_kernel<MT, WK, UW, UA, false, kFp32, true>,                               \
     gemm_decode_wide_kernel<MT, WK, UW, UA, false, kFp16, true>,                               \
-    gemm_decode_wide_kernel<MT, WK, UW, UA, false, kBf16, true>}}
+    gemm_decode_wide_kernel<MT, WK, UW, UA, false, kBf16, true>},                              \
+   {nullptr, nullptr, nullptr},                                                                \
+   {gemm_decode_wide_kernel<MT, WK, UW, UA, true, kFp32, true, 1, 16, true>,                   \
+    gemm_decode_wide_kernel<MT, WK, UW, UA, true, kFp16, true, 1, 16, true>,                   \
+    gemm_decode_wide_kernel<MT, WK, UW, UA, true, kBf16, true, 1, 16, true>},                  \
+   {gemm_decode_wide_kernel<MT, WK, UW, UA, false, kFp32, true, 1, 16, true>,                  \
+    gemm_decode_wide_kernel<MT, WK, UW, UA, false, kFp16, true, 1, 16, true>,                  \
+    gemm_decode_wide_kernel<MT, WK, UW, UA, false, kBf16, true, 1, 16, true>}}
 #define DECODE_WIDE_M8CFG(WK, UW, UA, NAME)                                                    \
   {4,                                                                                          \
    16,                                                                                         \
@@ -2775,8 +2795,18 @@ extern "C" int inferop_hip_gemm_w8a8_block_grouped(void* c, const uint8_t* a_q,
     // one workgroup per (16-row weight stripe, virtual M tile of the experts)
     if (16 * k > 0x7FFFFFFF || tmv > 65535) return hipErrorInvalidConfiguration;
     const int64_t per_wave = (k / 128 + cf.waves - 1) / cf.waves;
-    const KernelFn fn = per_wave <= wide_scale_cap() ? cf.fn_grp[di] : cf.fn_grp_alt[di];
-    hipLaunchKernelGGL(fn, dim3((unsigned)tn, (unsigned)launch_tmv), dim3(64 * cf.waves), 0, st, args);
+    const bool pre = per_wave <= wide_scale_cap();
+    // Masked experts of more than two tiles: this kernel is chosen for few rows
+    // per expert, so most of those tiles are empty, and a grid of two per
+    // expert whose workgroups walk on saves launching them (32 experts, N=4096,
+    // K=7168, max_m 128: 64 rows 205.6 -> 154.7 us, 200 rows 227.5 -> 176.4; max_m 64, 64 rows 162.8 -> 154.5).
+    // With a grid of every tile the walk's loop cost 1-6% (max_m 16 131.1 -> 133.4 us,
+    // 32 141.0 -> 147.5).
+    const bool walks = max_m > 0 && launch_tmv > 2 * experts;
+    const KernelFn fn = walks ? (pre ? cf.fn_walk[di] : cf.fn_walk_alt[di])
+                              : (pre ? cf.fn_grp[di] : cf.fn_grp_alt[di]);
+    hipLaunchKernelGGL(fn, dim3((unsigned)tn, (unsigned)(walks ? 2 * experts : launch_tmv)),
+                       dim3(64 * cf.waves), 0, st, args);
     return hipGetLastError();
   }
   int64_t grid = tn * launch_tmv;

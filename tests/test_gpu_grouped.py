@@ -243,14 +243,16 @@ def test_grouped_masked_layout(name):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("max_m", [1, 8, 16, 17])
+@pytest.mark.parametrize("max_m,k", [(1, 512), (8, 512), (16, 512), (17, 512), (70, 512),
+                                     (70, 16640)])
 @pytest.mark.parametrize("name", GROUPED)
-def test_grouped_masked_grid_holds_full_experts(name, max_m):
+def test_grouped_masked_grid_holds_full_experts(name, max_m, k):
     # the grid holds experts * ceil(max_m / tile rows) tiles at most: with every
-    # expert full (one count past max_m) the last expert's last tile is in it
+    # expert full (one count past max_m) the last expert's last tile is in it; at
+    # 70 rows wide decode workgroups walk on, with the scales preloaded and not
     device()
     counts = [max_m] * 5
-    n, k = 72, 512
+    n = 72
     aq, as_, bq, bs, offsets = _experts(counts, n, k, seed=31 + max_m)
     a3, s3 = _masked_inputs(counts, max_m, aq, as_, offsets)
     cfg = _cfg(name)
