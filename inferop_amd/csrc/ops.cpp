@@ -625,7 +625,8 @@ int quant_gemm_impl(void* c, void* q, void* scales, const void* x, int32_t dt, c
 // best: two 128x128 workgroups per CU up to 64 rows per expert, one 256x256
 // beyond (32 experts, N=4096, K=7168: 90 rows 217 -> 177 us, 128 rows 287 -> 197; 8
 // experts, 70 rows 83.6 -> 72.1), from 96 rows where the 256x256 tiles leave
-// three quarters of the CUs idle (32 experts, N=512, 90 rows 61.4 vs 67.1).
+// three quarters of the CUs idle (32 experts, N=512, 90 rows 61.4 vs 67.1) or K
+// is past what 32-bit offsets reach in 256 rows.
 // Where those tiles cover at most half of the CUs
 // (2 * experts * ceil(N / 256) <= CUs) every workgroup walks the whole K of
 // its one tile alone and the weights arrive at half the chip's rate or less:
@@ -654,7 +655,9 @@ int32_t select_grouped(int64_t m, int64_t launch_m, int64_t n, int64_t k, int64_
   if (avg > 8 && avg <= 24 && even && kg >= 24 && 2 * t256 <= cus && 32 * k <= 0x7FFFFFFF &&
       (launch_m + 31) / 32 + ne <= 65535)
     return kDwM32K4;
-  if (even) return avg <= 64 || (avg < 96 && 4 * t256 <= cus) ? kPerN128M128 : kPerN256M256;
+  const bool tall = 256 * k <= 0x7FFFFFFF;  // 256-row tiles can address their rows
+  if (even && (avg <= 64 || (avg < 96 && (4 * t256 <= cus || !tall)))) return kPerN128M128;
+  if (even) return kPerN256M256;
   if (avg < 16) return kPreN128M16S4;
   if (avg < 24) return kPreN128M32S4;
   if (avg < 64) return kPreN128M64S3;

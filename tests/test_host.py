@@ -456,3 +456,15 @@ def test_grouped_selection_short_k_and_few_tiles():
                                                                               exp)]
     assert msel(1024, 128, 16) == "dw_m32_k4_w2a2"
     assert msel(32768, 128, 16) == "per_n128_m128_w4"
+
+
+def test_grouped_selection_stays_within_a_kernel_k_limit():
+    # a tile's rows are addressed with 32-bit offsets: 65 to 95 rows per expert over a
+    # K that 256-row tiles cannot take run on 128-row tiles
+    names = [inferop_amd.gemm_config_name(i) for i in range(inferop_amd.gemm_num_configs())]
+    sel = lambda avg, n, k, e: names[inferop_amd.grouped_gemm_select(avg * e, n, k, e)]
+    longest = (0x7FFFFFFF // 256) // 256 * 256  # whole pairs of scale groups
+    for avg in (65, 80, 95):
+        assert sel(avg, 4096, longest, 8) == "per_n256_m256_w8"
+        assert sel(avg, 4096, longest + 256, 8) == "per_n128_m128_w4"
+        assert sel(avg, 4096, 0x7FFFFFFF // 128 // 256 * 256, 8) == "per_n128_m128_w4"
