@@ -72,7 +72,7 @@ __global__ __launch_bounds__(SPLIT ? 128 : 64) void topk_softmax_kernel(int32_t*
   // workgroup took 6.1 us against 5.5 us, at 4096 tokens the two are level
   __shared__ __attribute__((aligned(16))) float sp[kMaxExperts];
   __shared__ float sum;
-  const int lane = threadIdx.x & 63;
+  const int lane = SPLIT ? threadIdx.x & 63 : threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const bool adds = !SPLIT || wave == 1, selects = !SPLIT || wave == 0;
   const int t = blockIdx.x;
