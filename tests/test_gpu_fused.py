@@ -113,6 +113,40 @@ def test_silu_lds_tables_match_small_call_kernel(kind):
         assert np.array_equal(ss.view(np.uint32), s[r0:r1].view(np.uint32)), r0
 
 
+@pytest.mark.parametrize("kind", ["bf16", "fp16"])
+@pytest.mark.parametrize("tokens,d", [(1100, 4096), (1537, 17 * 128), (24593, 17 * 128),
+                                      (4096, 18432)])
+def test_silu_lds_walk_matches_small_call_kernel(kind, tokens, d):
+    # a workgroup of the LDS-table kernel goes through the groups in strides,
+    # carrying (token, group of the token) forward by additions: on 256 CUs one or
+    # two steps of 64 groups each (fp16) at 35200 groups, one at 26129; three to
+    # five (bf16) or eight to twelve (fp16) above 262144 groups, 16 steps per CU,
+    # where bf16 launches twice the workgroups; with 17, 32 and 144 groups per
+    # token, the last step short or full.  Rows are independent, so the same rows in calls below 16384 groups,
+    # which the small-call kernel takes, give the same bits.
+    device()
+    g = torch.Generator(device="cuda:0")
+    g.manual_seed(tokens)
+    gu = 2.0 * torch.randn((tokens, 2 * d), device="cuda:0", generator=g)
+    gu[::7, ::5] *= 64.0  # gates past the slice too
+    gu[1::7, ::5] *= 2.0 ** -12
+    gu = gu.to(torch.bfloat16 if kind == "bf16" else torch.float16)
+
+    def call(part):
+        n = part.shape[0]
+        q = torch.full((n, d), 0xA5, dtype=torch.uint8, device="cuda:0")
+        s = torch.full((n, d // 128), -1.0, dtype=torch.float32, device="cuda:0")
+        assert ia.silu_and_mul_quant_fp8(q, s, part, getattr(DT, kind), n, d) == 0
+        return q, s
+
+    q, s = call(gu)
+    rows = 16383 // (d // 128)
+    for r0 in range(0, tokens, rows):
+        qs, ss = call(gu[r0:r0 + rows])
+        assert torch.equal(qs, q[r0:r0 + rows]), r0
+        assert torch.equal(ss, s[r0:r0 + rows]), r0
+
+
 @pytest.mark.parametrize("kind", ["bf16", "fp16", "fp32"])
 @pytest.mark.parametrize("shape", [(1, 2048), (64, 18432 // 8), (77, 7168 // 4), (16411, 128),
                                    (4096, 18432 // 8)])
