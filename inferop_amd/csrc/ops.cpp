@@ -341,13 +341,17 @@ GemmChoice select_gemm(int64_t m, int64_t n, int64_t k, int cus) {
   // CU's tiles and drains their stores in the background); the tiles of its
   // last, partial round are cut along K into up to 8 pieces that run at once
   // (their partials added by a second kernel) when the round time saved,
-  // kg * (1 - 1/S) group-rounds, exceeds the cost of writing and re-reading
-  // tail * S partial tiles of 256 KB (at ~5 TB/s, ~0.026 group-rounds each)
-  // plus ~2.4 group-rounds of fixed cost (a group-round of 256x256 tiles
-  // takes ~2.05 us on 256 CUs).  Measured on MI355X: M=4096, N=4608,
-  // K=7168 (288 tiles) 177 -> 138 us with S=8 (128x128 tiles: 161 us);
-  // M=512, N=7168, K=18432 (56 tiles) 220 -> 89 us with S=4 (128x128: 115-132
-  // us); M=8192, N=7168, K=2048 (896 tiles) 139 us unsplit, 143 us with S=2.
+  // kg * (1 - 1/S) group-rounds, exceeds the cost of the pieces: writing and
+  // re-reading tail * S partial tiles of 256 KB (0.035 group-rounds each), the
+  // second launch with the pipeline's filling and draining (6), and 0.15 per
+  // scale group, as the pieces of few tiles run slower than whole rounds.  A
+  // group-round of 256x256 tiles takes 1.45-1.9 us on 256 CUs.  Fitted to 195
+  // pairs of split and unsplit calls (16 to 128 tiles left, S 2 to 8, K/128 from
+  // 8 to 96); on 680 other pairs, of those that reach it (a whole round of tiles
+  // or K/128 >= 48), the slower of the two is taken by 2% at most (4% seen with a
+  // ragged last row of tiles).  Same box, unsplit and split, us: M=4096, N=4608 (288 tiles, S=8) K=2048 53.8 / 61.0,
+  // K=3072 78.3 / 74.0, K=8192 187.8 / 146.6; N=6144 (384, S=2) K=4096 110.6 /
+  // 117.9, K=8192 212.0 / 197.4; M=512, N=7168, K=12288 (56, S=4) 146 / 73.
   const int64_t t256 = ((n + 255) / 256) * ((m + 255) / 256);
   const int64_t t128 = ((n + 127) / 128) * ((m + 127) / 128);
   auto tail_split = [&]() -> int32_t {
@@ -358,7 +362,7 @@ GemmChoice select_gemm(int64_t m, int64_t n, int64_t k, int cus) {
     if (sp > kg / 2) sp = kg / 2;
     if (sp < 2) return 1;
     const double saved = (double)kg * (1.0 - 1.0 / (double)sp);
-    const double cost = (double)(tail * sp) * 0.0256 + 2.4;
+    const double cost = 6.0 + 0.035 * (double)(tail * sp) + 0.15 * (double)kg;
     return saved > cost ? int32_t(sp) : 1;
   };
   // at least one whole round of 256x256 tiles, or a long K: the persistent

@@ -254,6 +254,16 @@ def test_gemm_selection_covers_configs():
     # persistent 256x256 tiles cut along K (configs[4] M=1000)
     assert sel(1000, 4672, 7168) == ("per_n256_m256_w8", 3)
     assert sel(1024, 7168, 2048) == ("pre_n128_m128_w4_s2", 1)
+    # the tiles of a partial last round are cut along K where the round time
+    # saved exceeds what the pieces cost: from about 24 scale groups with 32 tiles
+    # left, 48 with 128
+    assert sel(4096, 4608, 1536) == ("per_n256_m256_w8", 1)
+    assert sel(4096, 4608, 2560) == ("per_n256_m256_w8", 1)
+    assert sel(4096, 4608, 3072) == ("per_n256_m256_w8", 8)
+    assert sel(4096, 6144, 5120) == ("per_n256_m256_w8", 1)
+    assert sel(4096, 6144, 8192) == ("per_n256_m256_w8", 2)
+    assert sel(3000, 7168, 2048) == ("per_n256_m256_w8", 1)
+    assert sel(512, 7168, 12288) == ("per_n256_m256_w8", 4)
     # 256x256 prefill tiles run on the persistent kernel when K / 128 is even,
     # on the one-tile-per-workgroup kernel otherwise
     assert names[inferop_amd.gemm_select(4096, 7168, 16384)[0]] == "per_n256_m256_w8"
