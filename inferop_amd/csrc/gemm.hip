@@ -533,10 +533,11 @@ __host__ __device__ constexpr int wide_scale_cap() { return 16; }
 // fixup.
 //
 // AR = 8 (one activation tile, M <= 8 rows per workgroup): a tile is 8 rows,
-// one load per group instead of two; the MFMA's other 8 columns read stale
-// LDS and their outputs are never stored or summed into stored outputs (each
-// output column of the MFMA depends only on its own activation row).  Grouped
-// tiles choose it per workgroup, by the rows their expert has in the tile.
+// one load per group instead of two; the MFMA's other 8 columns read those
+// rows again and their outputs are never stored or summed into stored outputs
+// (each output column of the MFMA depends only on its own activation row).
+// Grouped tiles choose it per workgroup, by the rows their expert has in the
+// tile.
 
 // LDS bytes of one wave: its two rings and the preloaded scales.
 template <int MT, int UW, int UA, bool PRE, int NT, int AR>
@@ -745,8 +746,9 @@ __global__ __launch_bounds__(64 * WK) void gemm_decode_wide_kernel(GemmArgs a) {
   const int n0 = blockIdx.x * (16 * NT);
   if constexpr (GROUPED) {
     // A tile of at most 8 rows of its expert takes an 8-row activation tile
-    // and, in the same LDS, rings one group deeper: MoE decode steps give an
-    // expert a few rows.  32 experts, 64 rows, N=4096, K=7168: 140.2 -> 133.5 us;
+    // and, for the LDS that saves (512 bytes a wave more without the scale
+    // preload), rings one group deeper: MoE decode steps give an expert a few
+    // rows.  32 experts, 64 rows, N=4096, K=7168: 140.2 -> 133.5 us;
     // 8 experts of 5 rows 45.1 -> 41.6, with N=7168, K=2048 33.8 -> 32.8.
     constexpr bool kShort = MT == 1 && UW == UA;
     constexpr int kWave = wide_wave_bytes<MT, UW, UA, PRE, NT, 16>();
@@ -2133,7 +2135,8 @@ struct CfgEntry {
   KernelFn fn_grp_alt[3];
   // persistent (kind 3): the reduction of cut tail tiles
   void (*fn_tail[3])(GemmArgs, int, int);
-  // wide decode (kind 4): fn_grp and fn_grp_alt walking a lower grid
+  // wide decode (kind 4): fn_grp and fn_grp_alt walking a lower grid, where built
+  // (else null)
   KernelFn fn_walk[3];
   KernelFn fn_walk_alt[3];
 };
@@ -2176,7 +2179,7 @@ struct CfgEntry {
    {gemm_decode_wide_kernel<MT, WK, UW, UA, false, kFp32>,                                     \
     gemm_decode_wide_kernel<MT, WK, UW, UA, false, kFp16>,                                     \
     gemm_decode_wide_kernel<MT, WK, UW, UA, false, kBf16>}}
-#define DECODE_WIDE_GCFG(MT, WK, UW, UA, NAME)                                                 \
+#define DECODE_WIDE_GCFG(MT, WK, UW, UA, NAME, ...)                                            \
   {4,                                                                                          \
    16,                                                                                         \
    16 * MT,                                                                                    \
@@ -2195,12 +2198,15 @@ struct CfgEntry {
     gemm_decode_wide_kernel<MT, WK, UW, UA, false, kFp16, true>,                               \
     gemm_decode_wide_kernel<MT, WK, UW, UA, false, kBf16, true>},                              \
    {nullptr, nullptr, nullptr},                                                                \
+   __VA_ARGS__}
+// the walking forms, of the configurations that the masked choice returns
+#define DECODE_WIDE_WALK(MT, WK, UW, UA)                                                       \
    {gemm_decode_wide_kernel<MT, WK, UW, UA, true, kFp32, true, 1, 16, true>,                   \
     gemm_decode_wide_kernel<MT, WK, UW, UA, true, kFp16, true, 1, 16, true>,                   \
     gemm_decode_wide_kernel<MT, WK, UW, UA, true, kBf16, true, 1, 16, true>},                  \
    {gemm_decode_wide_kernel<MT, WK, UW, UA, false, kFp32, true, 1, 16, true>,                  \
     gemm_decode_wide_kernel<MT, WK, UW, UA, false, kFp16, true, 1, 16, true>,                  \
-    gemm_decode_wide_kernel<MT, WK, UW, UA, false, kBf16, true, 1, 16, true>}}
+    gemm_decode_wide_kernel<MT, WK, UW, UA, false, kBf16, true, 1, 16, true>}
 #define DECODE_WIDE_M8CFG(WK, UW, UA, NAME)                                                    \
   {4,                                                                                          \
    16,                                                                                         \
@@ -2280,12 +2286,12 @@ const CfgEntry kCfgs[] = {
     PERSIST_PP_CFG("per_n256_m256_w8"),
     PERSIST_CFG(256, 128, 4, 2, "per_n256_m128_w8"),
     PERSIST_CFG(128, 128, 2, 2, "per_n128_m128_w4"),
-    DECODE_WIDE_GCFG(4, 4, 2, 2, "dw_m64_k4_w2a2"),
+    DECODE_WIDE_GCFG(4, 4, 2, 2, "dw_m64_k4_w2a2", {}, {}),
     DECODE_WIDE_CFG(4, 2, 4, 2, "dw_m64_k2_w4a2"),
-    DECODE_WIDE_GCFG(2, 4, 2, 2, "dw_m32_k4_w2a2"),
+    DECODE_WIDE_GCFG(2, 4, 2, 2, "dw_m32_k4_w2a2", DECODE_WIDE_WALK(2, 4, 2, 2)),
     DECODE_WIDE_CFG(1, 2, 8, 8, "dw_m16_k2_w8a8"),
-    DECODE_WIDE_GCFG(1, 8, 3, 3, "dw_m16_k8_w3a3"),
-    DECODE_WIDE_GCFG(1, 4, 3, 3, "dw_m16_k4_w3a3"),
+    DECODE_WIDE_GCFG(1, 8, 3, 3, "dw_m16_k8_w3a3", {}, {}),
+    DECODE_WIDE_GCFG(1, 4, 3, 3, "dw_m16_k4_w3a3", DECODE_WIDE_WALK(1, 4, 3, 3)),
     DECODE_WIDE_CFG(1, 8, 2, 2, "dw_m16_k8_w2a2"),
     DECODE_WIDE_NCFG(4, 4, 4, 2, 2, "dw_n64_m64_k4_w2a2"),
     DECODE_WIDE_NCFG(2, 4, 4, 2, 2, "dw_n32_m64_k4_w2a2"),
@@ -2799,10 +2805,17 @@ extern "C" int inferop_hip_gemm_w8a8_block_grouped(void* c, const uint8_t* a_q,
     // Masked experts of more than two tiles: this kernel is chosen for few rows
     // per expert, so most of those tiles are empty, and a grid of two per
     // expert whose workgroups walk on saves launching them (32 experts, N=4096,
-    // K=7168, max_m 128: 64 rows 205.6 -> 154.7 us, 200 rows 227.5 -> 176.4; max_m 64, 64 rows 162.8 -> 154.5).
-    // With a grid of every tile the walk's loop cost 1-6% (max_m 16 131.1 -> 133.4 us,
-    // 32 141.0 -> 147.5).
-    const bool walks = max_m > 0 && launch_tmv > 2 * experts;
+    // K=7168, max_m 128: 64 rows 205.6 -> 154.7 us, 200 rows 227.5 -> 176.4; max_m
+    // 64, 64 rows 162.8 -> 154.5; 8 experts, 16 rows, N=7168, K=2048, max_m 256 100.4
+    // -> 36.9).  With a grid of every tile the walk's loop cost 1-6% (max_m 16 131.1
+    // -> 133.4 us, 32 141.0 -> 147.5).  It loses 2-8% where every
+    // expert is full against a hint of 8 rows or fewer (32 experts, max_m 48
+    // 564 -> 578 us, 128 1486 -> 1588, 256 2954 -> 3170; 16 experts, N=2048,
+    // K=1536, max_m 48 47.3 -> 49.1); one full expert among short ones still
+    // gains (max_m 128 272 -> 200).  Walking runs of neighbouring tiles, alone or
+    // eight rows side by side, was 1-6% faster on the longest of these walks and
+    // up to 11% slower on the short ones.
+    const bool walks = cf.fn_walk[di] && max_m > 0 && launch_tmv > 2 * experts;
     const KernelFn fn = walks ? (pre ? cf.fn_walk[di] : cf.fn_walk_alt[di])
                               : (pre ? cf.fn_grp[di] : cf.fn_grp_alt[di]);
     hipLaunchKernelGGL(fn, dim3((unsigned)tn, (unsigned)(walks ? 2 * experts : launch_tmv)),
