@@ -1381,8 +1381,8 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_persist_kernel(GemmArgs a) 
   // tile up, so that in an expert's last tile, which often ends early, the
   // waves with no rows left are the loading ones (0 .. NL-1); they skip the
   // multiply and only issue loads, and the busy wave on each SIMD has the
-  // matrix core to itself (32 experts, N=4096, K=7168, 4096 rows on 256x256
-  // tiles: 270.7 -> 250 us; 2048 rows 242 -> 220 us).  With one wave per
+  // matrix core to itself (32 experts, N=4096, K=7168 on 256x128 tiles: 64 rows
+  // 212 -> 191 us, 1024 rows 205 -> 191, 4096 rows 301 -> 292).  With one wave per
   // SIMD (128x128 tiles) nothing is gained and it measured 4% slower; the
   // plain GEMM keeps top-down rows (the reversed order spills 64 more
   // registers there).
@@ -1453,16 +1453,17 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_persist_kernel(GemmArgs a) 
     const uint8_t* bB = st;
     const uint8_t* bA = st + kOffA;
     const float* sA = reinterpret_cast<const float*>(st + kOffSA);
-    // Plain GEMM: the weight operand of slice i+1 is read while slice i is
-    // multiplied, so its LDS latency is not waited out before the slice's
-    // first MFMA (256x256 tiles: 7168x16384 470 -> 459 us, 24576x1536
-    // 167 -> 163 us), and the first slice's operands are read ahead of the
-    // scales, so the group's first MFMA does not wait for the scale reads
-    // (LDS returns in order; 7168x16384 471 -> 468 us).  The grouped forms
-    // keep the read in the slice: with the prefetch they lost time (32
-    // experts, N=4096, K=7168: 2 rows per expert on 128x128 tiles 152 -> 177
-    // us, 128 rows on 256x256 254 -> 261 us).
-    constexpr bool kPrefetch = !GROUPED;
+    // Plain GEMM on 256x128 tiles: the weight operand of slice i+1 is read while
+    // slice i is multiplied, so its LDS latency is not waited out before the
+    // slice's first MFMA, and the first slice's operands are read ahead of the
+    // scales, so the group's first MFMA does not wait for the scale reads (LDS
+    // returns in order): 7168x16384 605 -> 585 us, 24576x1536 202 -> 198.  On 128x128
+    // tiles, two workgroups per CU, it costs time, so the read stays in the
+    // slice: M=384, N=4096, K=7168 36.4 us with it, 34.8 without, M=512, N=6144,
+    // K=9216 73.7 and 68.7, M=300, N=6144, K=7168 44.6 and 40.9; and so in the grouped
+    // forms (32 experts, N=4096, K=7168, 2 rows per expert on 128x128 tiles 187.7 and
+    // 165.0).
+    constexpr bool kPrefetch = !GROUPED && BN > 128;
     i32x8 bnext{};
     if constexpr (kPrefetch) bnext = lds_operand(bB, wn * TN + rsub, c0);
     i32x8 aop[SM];
@@ -1474,9 +1475,9 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_persist_kernel(GemmArgs a) 
     for (int j = 0; j < SM; ++j) sab[j] = sA[wm * TM + 16 * j + rsub] * sbC;
     // Plain GEMM: all SM MFMAs of a slice before their promotion FMAs, so
     // each partial is read several MFMAs after it was issued, with no wait
-    // states (24576x1536 188.7 -> 184.7 us, 7168x16384 472.7 -> 465.7,
-    // 4096^3 74.9 -> 72.7; same box, alternating builds).  The grouped forms,
-    // which hold more state, keep pairs: four spilled 16-32 more bytes there.
+    // states (measured while this form ran 256x256 tiles too: 24576x1536 188.7 ->
+    // 184.7 us, 4096^3 74.9 -> 72.7).  The grouped forms, which hold more state,
+    // keep pairs: four spilled 16-32 more bytes there.
     constexpr int PJ = (GROUPED && SM >= 4) ? 2 : SM;
 #pragma unroll
     for (int i = 0; i < SN; ++i) {
