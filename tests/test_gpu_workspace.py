@@ -134,3 +134,26 @@ def test_default_stream_is_torchs_current_one():
         assert seen[0][0] == seen[0][1]
     assert ops._stream(None) == torch.cuda.current_stream().cuda_stream
     assert ops._stream(side) == side.cuda_stream and ops._stream(17) == 17
+
+
+@pytest.mark.gpu
+def test_default_stream_in_a_forked_child_is_the_null_stream():
+    # a child forked after the handle is read directly has no device: the null
+    # stream, and no call into the device runtime.  The child does nothing else.
+    import os
+
+    from inferop_amd import ops
+
+    device()
+    with torch.cuda.stream(torch.cuda.Stream()):
+        assert ops._stream(None) != 0
+        assert ops._current_stream is not ops._first_current_stream
+        pid = os.fork()
+        if pid == 0:
+            code = 1
+            try:
+                code = 0 if ops._stream(None) == 0 else 2
+            finally:
+                os._exit(code)
+        assert os.waitstatus_to_exitcode(os.waitpid(pid, 0)[1]) == 0
+        assert ops._stream(None) != 0
