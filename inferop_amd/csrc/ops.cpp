@@ -5,6 +5,7 @@
 // device introspection) and the gfx950 tile selection that replaces the
 // reference's SM-version switch (kernels/gemm/w8a8_block_fp8.cu:142-159).
 // Kernels are reached through the thin C launch layer in hip_launch.h.
+#include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -620,10 +621,16 @@ int quant_gemm_impl(void* c, void* q, void* scales, const void* x, int32_t dt, c
 // 153 us vs 171 us on the persistent 128x128 tiles, 8 rows 163 vs 171 us; at
 // 16 rows 243 vs 174 us), except over a short K (up to 20 scale groups, even)
 // with a 256x256 tile per CU or more, where a stripe's workgroup spends its time
-// filling and draining its rings and the persistent kernels take over from 2
-// rows per expert (16 experts, N=7168, K=2048: 2 rows 60.1 -> 51.2 us, 8 rows
-// 64.6 -> 52.0; 32 experts, N=4096, K=2304: 70.9 -> 60.7, 78.4 -> 61.8; at 32
-// groups the stripes stay ahead, 32 experts, N=7168, K=4096, 8 rows: 188 vs 233).
+// filling and draining its rings: there the persistent 128x128 tiles take over
+// from 2 rows per expert, the later the longer K is and the less the last round
+// of their tiles (two per CU) fills.  Their time over the stripe kernel's, rows
+// spread at random, is about (0.47 + 0.0225 K/128) * (1 - 0.02 (rows - 2)) over the
+// part of the rounds that tiles fill to the power 0.6 (fitted to 676 pairs, 4 to
+// 20 groups, 0.62 to 1 of the rounds filled, 2 to 8 rows): 16 experts, N=7168,
+// K=2048 (0.88), 2 rows 58.0 -> 52.9 us, 8 rows 65.6 -> 52.1; 64 experts, N=1536
+// (0.75), 4 rows K=2048 52.7 -> 49.7, K=2560 1.04 times the stripes' time; N=1280,
+// K=2560 (0.62), 2 to 6 rows 1.16 to 1.31 times; at 32 groups the stripes stay
+// ahead (32 experts, N=7168, K=4096, 8 rows: 188 vs 233).
 // Beyond that, with an even K / 128, the persistent kernels, whose load
 // pipeline runs on across a workgroup's tiles, stream the experts' weights
 // best: two 128x128 workgroups per CU up to 64 rows per expert, one 256x256
@@ -638,7 +645,11 @@ int quant_gemm_impl(void* c, void* q, void* scales, const void* x, int32_t dt, c
 // 24 scale groups up (8 experts, N=1000, K=7168, 16 rows 52.9 -> 15.1 us; 8
 // experts, N=4096, K=7168: 12 rows 69.4 -> 51.7, 24 rows 70.6 -> 60.2; 16
 // experts, N=2048, K=7168, 24 rows 71.1 -> 67.5; over 12 groups it loses, 16
-// experts, N=2048, K=1536, 16 rows 19.2 vs 20.3).  With an odd K / 128 the
+// experts, N=2048, K=1536, 16 rows 19.2 vs 20.3).  Beyond 24 rows some expert of a
+// random routing passes 32 rows and takes a second tile, which reads the
+// weights again: 8 experts, N=4096, K=7168: 25 rows 60.2 vs 70.2 us on the
+// persistent tiles, 28 rows 72.4 vs 70.8, 32 rows 87.5 vs 72.6 (64-row wide tiles
+// 90-92).  With an odd K / 128 the
 // tiled kernels: 16-row tiles below 16 rows per expert, 32-row below 24,
 // 64-row three-stage below 64, 128x128 beyond.
 // m: the rows the tile choice is made for (masked layout: the expected rows
@@ -653,7 +664,13 @@ int32_t select_grouped(int64_t m, int64_t launch_m, int64_t n, int64_t k, int64_
   const int64_t kg = k / 128;
   const bool even = kg % 2 == 0;
   const int64_t t256 = num_experts * ((n + 255) / 256);  // one 256-row tile per expert
-  const bool short_k = even && kg <= 20 && t256 >= cus && avg >= 2;
+  bool short_k = avg >= 2 && avg <= 8 && even && kg <= 20 && t256 >= cus;
+  if (short_k) {
+    const int64_t t128 = num_experts * ((n + 127) / 128), slots = 2 * (int64_t)cus;
+    const double fill = (double)t128 / (double)((t128 + slots - 1) / slots * slots);
+    short_k = (0.47 + 0.0225 * (double)kg) * (1.0 - 0.02 * (double)(avg - 2)) <=
+              std::pow(fill, 0.6);
+  }
   if (avg <= 8 && !short_k && 16 * k <= 0x7FFFFFFF && (launch_m + 15) / 16 + ne <= 65535)
     return kDwM16K4;
   if (avg > 8 && avg <= 24 && even && kg >= 24 && 2 * t256 <= cus && 32 * k <= 0x7FFFFFFF &&

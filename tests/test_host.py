@@ -478,3 +478,19 @@ def test_grouped_selection_stays_within_a_kernel_k_limit():
         assert sel(avg, 4096, longest, 8) == "per_n256_m256_w8"
         assert sel(avg, 4096, longest + 256, 8) == "per_n128_m128_w4"
         assert sel(avg, 4096, 0x7FFFFFFF // 128 // 256 * 256, 8) == "per_n128_m128_w4"
+
+
+def test_grouped_selection_short_k_by_filled_rounds():
+    # a short K goes to the persistent 128x128 tiles where their last round (two
+    # tiles per CU, 512 slots) is full enough for K and the rows per expert
+    names = [inferop_amd.gemm_config_name(i) for i in range(inferop_amd.gemm_num_configs())]
+    sel = lambda avg, n, k, e: names[inferop_amd.grouped_gemm_select(avg * e, n, k, e)]
+    stripes, tiles = "dw_m16_k4_w3a3", "per_n128_m128_w4"
+    assert [sel(2, n, 2048, 64) for n in (1280, 1536, 1792, 2048)] == [stripes, tiles, tiles,
+                                                                       tiles]
+    assert [sel(2, n, 2560, 64) for n in (1280, 1536, 2048, 2304)] == [stripes, stripes, tiles,
+                                                                       stripes]
+    assert [sel(avg, 1536, 18 * 128, 64) for avg in (1, 2, 4, 8)] == [stripes, stripes, tiles,
+                                                                      tiles]
+    assert sel(2, 1280, 1024, 64) == tiles
+    assert [sel(avg, 1280, 2560, 64) for avg in (2, 4, 8, 9)] == [stripes, stripes, stripes, tiles]
