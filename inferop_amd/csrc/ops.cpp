@@ -415,7 +415,7 @@ GemmChoice select_gemm(int64_t m, int64_t n, int64_t k, int cus) {
   // 128x128 tiles run unsplit, some CUs holding two), over a K of 48 scale
   // groups or more: the persistent 256x256 tiles, all in their first, partial
   // round and cut along K, read a quarter fewer operand bytes per CU
-  // (configs[4] M=1000, N=4672, K=7168: 76 tiles cut in 3, 68.2 -> 59.5 us;
+  // (M=1000, N=4672, K=7168: 76 tiles cut in 3, 68.2 -> 59.5 us;
   // the 128x128 tiles put two on 40 CUs)
   if (kg % 2 == 0 && kg >= 48 && t256 < cus && t128 >= cus) {
     const int32_t s = tail_split();

@@ -54,7 +54,7 @@ def rng(seed: int, stream: int = 0) -> np.random.Generator:
 def activations(m: int, k: int, seed: int, dist: str = "normal") -> np.ndarray:
     """fp32 activations before 16-bit packing.
 
-    normal: N(0, 1).  stress (config 4): 4 * Student-t(3), 1% of 1x128 groups
+    normal: N(0, 1).  stress: 4 * Student-t(3), 1% of 1x128 groups
     set to zero, 0.1% of elements set to +-1792 (= 448 * 4, the largest
     outliers the scaled distribution is quoted with)."""
     g = rng(seed, 1)

@@ -53,7 +53,7 @@ def bf16_ulp(v: np.ndarray) -> np.ndarray:
 
 def assert_gemm_close(got: np.ndarray, ref: np.ndarray, what: str = ""):
     """max |got - ref| <= 1e-2 * rms(ref) + one bf16 ulp of |ref| (elementwise),
-    the tolerance BASELINE.json states for the blockwise GEMM."""
+    the blockwise GEMM's tolerance."""
     got = got.astype(np.float64)
     ref = ref.astype(np.float64)
     assert got.shape == ref.shape

@@ -1,5 +1,5 @@
 """GPU blockwise-FP8 GEMM parity with the oracle (reference.cpp:93-110, fp64
-accumulation) on all five BASELINE.json configs, to the stated tolerance
+accumulation) on the decode, prefill, M-sweep and ragged workloads, to the tolerance
 max|err| <= 1e-2 * rms(C_ref) + 1 bf16 ulp."""
 import os
 
@@ -38,7 +38,7 @@ def _host_case(m, n, k, seed, dist="normal"):
 
 @pytest.mark.gpu
 def test_config0_golden_end_to_end():
-    # BASELINE config 0, expected output written by the reference's own code:
+    # M=16, N=512, K=1024, expected output written by the reference's own code:
     # GPU quantizer on the bf16 activations, then the GPU GEMM
     device()
     g = np.load(os.path.join(GOLDEN, "config0.npz"))

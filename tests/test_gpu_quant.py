@@ -111,7 +111,7 @@ def test_quant_rejected_shapes_leave_outputs_untouched():
 
 @pytest.mark.gpu
 def test_quant_large_whole_tensor_and_roundtrip():
-    # M=4096, K=16384 (config 2's largest K): every byte and scale against the
+    # M=4096, K=16384 (the largest prefill K): every byte and scale against the
     # oracle, and the size-independent round-trip bound on top
     device()
     m, k = 4096, 16384

@@ -3,7 +3,7 @@ no counterpart in the reference: its decode step is quant_fp8_per_token_group,
 ops.h:64-65, then w8a8_block_fp8_gemm, ops.h:81-84).  It must write the very
 bytes the two calls write: q / scales equal to the quantizer's (and so to the
 oracle's, reference.cpp:65-80) and C equal bit for bit to the GEMM on them --
-on every configs[1] shape (one launch at M = 1, two at M = 16 and 64), on
+on every decode-step shape (one launch at M = 1, two at M = 16 and 64), on
 fp16 and fp32 activations, ragged N, and the quantizer's edge groups (NaN,
 Inf, zero, subnormal) -- and C within the GEMM tolerance of the oracle."""
 import numpy as np

@@ -251,7 +251,7 @@ def test_gemm_selection_covers_configs():
     assert sel(160, 18432, 7168) == ("per_n256_m256_w8", 3)
     assert sel(160, 24576, 1536) == ("pre_n128_m128_w4_s2", 1)
     # fewer 256x256 tiles than CUs, at least as many 128x128 tiles, a long K:
-    # persistent 256x256 tiles cut along K (configs[4] M=1000)
+    # persistent 256x256 tiles cut along K
     assert sel(1000, 4672, 7168) == ("per_n256_m256_w8", 3)
     assert sel(1024, 7168, 2048) == ("pre_n128_m128_w4_s2", 1)
     # the tiles of a partial last round are cut along K where the round time
